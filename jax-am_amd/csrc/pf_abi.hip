@@ -1,10 +1,9 @@
 // C ABI of libpfhip.so (include/pfhip.h): single-instance step, temperature,
-// initial condition, argmax and FP64 diagnostics.  The batched engine is in
+// and initial condition.  Argmax and the diagnostics are in pf_reduce.hip, the batched engine in
 // pf_batch.hip, the register-tiled instantiations in pf_inst_*.hip.
 #include <math.h>
 #include <string.h>
 
-#include <mutex>
 #include <string>
 #include <vector>
 
@@ -293,194 +292,6 @@ __global__ __launch_bounds__(256) void voronoi_kernel(const double* __restrict__
   if (c < n) out[c] = gori ? gori[bi] : bi;
 }
 
-// numpy.argmax semantics: first maximum; a NaN is the maximum (first NaN wins)
-template <class TS>
-__device__ __forceinline__ int cell_argmax(const TS* __restrict__ row, int k) {
-  using TC = typename Traits<TS>::TC;
-  TC best = to_tc(row[0]);
-  int bi = 0;
-  if (best != best) return 0;
-  for (int i = 1; i < k; ++i) {
-    const TC v = to_tc(row[i]);
-    if (v != v) return i;
-    if (v > best) {
-      best = v;
-      bi = i;
-    }
-  }
-  return bi;
-}
-
-template <class TS>
-__global__ __launch_bounds__(256) void argmax_kernel(const TS* __restrict__ eta, long long n_cells, int k,
-                                                    int32_t* __restrict__ out) {
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= n_cells) return;
-  out[c] = cell_argmax(eta + c * k, k);
-}
-
-// ---- deterministic FP64 diagnostics
-constexpr int RB = 256;          // threads per reduction block
-constexpr int RMAXK = 256;       // histogram capacity (K <= RMAXK)
-constexpr int NF = 4;            // F_local, F_grad, max T, sum eta
-constexpr int NI = 3;            // changed, liquid, nonfinite
-
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-__device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-  return v;
-}
-__device__ __forceinline__ long long wave_sum_i(long long v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
-static int reduce_blocks(long long n) {
-  long long b = (n + RB * 8 - 1) / (RB * 8);
-  if (b < 1) b = 1;
-  if (b > 2048) b = 2048;
-  return (int)b;
-}
-static const long long kColRows = 4096;
-
-template <class TS>
-__global__ __launch_bounds__(RB) void reduce_cells_kernel(const StepDev a, const TS* __restrict__ eta,
-                                                         const int32_t* __restrict__ argmax0, double t, double m_g,
-                                                         double gamma, double ad_hoc, double half_kappa_ad,
-                                                         long long per_block, double* __restrict__ part_f,
-                                                         long long* __restrict__ part_i) {
-  using TC = typename Traits<TS>::TC;
-  __shared__ int hist[RMAXK];
-  __shared__ double sf[RB / 64][NF];
-  __shared__ long long si[RB / 64][NI];
-  const int K = a.k;
-  const int nx = a.nx, ny = a.ny, nz = a.nz;
-  const long long n = (long long)nz * ny * nx;
-  for (int i = threadIdx.x; i < K; i += RB) hist[i] = 0;
-  __syncthreads();
-  const long long c0 = (long long)blockIdx.x * per_block;
-  const long long c1 = min(n, c0 + per_block);
-  double f_loc = 0.0, f_grad = 0.0, tmax = -INFINITY, esum = 0.0;
-  long long changed = 0, liquid = 0, nonfinite = 0;
-  const double ih2[3] = {a.ihx2, a.ihy2, a.ihz2};
-  for (long long c = c0 + threadIdx.x; c < c1; c += RB) {
-    const int ix = (int)(c % nx), iy = (int)((c / nx) % ny), iz = (int)(c / ((long long)nx * ny));
-    const TS* row = eta + c * K;
-    double S = 0.0, s4 = 0.0, q = 0.0;
-    for (int i = 0; i < K; ++i) {
-      const double v = (double)to_tc(row[i]);
-      const double v2 = v * v;
-      S += v2;
-      s4 += v2 * v2;
-      q += v2 * v2 / 4.0 - v2 / 2.0;
-      esum += v;
-      if (!isfinite(v)) ++nonfinite;
-    }
-    const double T = cell_temperature(a, ix, iy, iz, c, t);
-    const double Tc = T > a.T_clip ? a.T_clip : T;
-    const double x = a.theta * (Tc / a.T_l - 1.0);
-    const double zeta = 0.5 * (1.0 - tanh(x));
-    const double omz = 1.0 - zeta;
-    // allen_cahn.py:45-48 with sum_ij (eta_i eta_j)^2 = S^2
-    f_loc += m_g * (q + gamma * (S * S - s4) + omz * omz * S) / ad_hoc;
-    const long long nb[3] = {ix + 1 < nx ? c + 1 : -1, iy + 1 < ny ? c + nx : -1,
-                             iz + 1 < nz ? c + (long long)nx * ny : -1};
-    for (int d = 0; d < 3; ++d) {
-      if (nb[d] < 0) continue;
-      const TS* r2 = eta + nb[d] * K;
-      double g = 0.0;
-      for (int i = 0; i < K; ++i) {
-        const double df = (double)to_tc(r2[i]) - (double)to_tc(row[i]);
-        g += df * df;
-      }
-      f_grad += g * ih2[d];
-    }
-    const int am = cell_argmax(row, K);
-    atomicAdd(&hist[am], 1);
-    if (argmax0 && argmax0[c] != am) ++changed;
-    if (T >= a.T_l) ++liquid;
-    tmax = fmax(tmax, T);
-  }
-  f_grad *= half_kappa_ad;
-  // fixed-order block reduction: wave butterflies, then waves in index order
-  f_loc = wave_sum(f_loc);
-  f_grad = wave_sum(f_grad);
-  tmax = wave_max(tmax);
-  esum = wave_sum(esum);
-  changed = wave_sum_i(changed);
-  liquid = wave_sum_i(liquid);
-  nonfinite = wave_sum_i(nonfinite);
-  const int w = threadIdx.x / 64;
-  if ((threadIdx.x & 63) == 0) {
-    sf[w][0] = f_loc;
-    sf[w][1] = f_grad;
-    sf[w][2] = tmax;
-    sf[w][3] = esum;
-    si[w][0] = changed;
-    si[w][1] = liquid;
-    si[w][2] = nonfinite;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double r[NF] = {0.0, 0.0, -INFINITY, 0.0};
-    long long ri[NI] = {0, 0, 0};
-    for (int j = 0; j < RB / 64; ++j) {
-      r[0] += sf[j][0];
-      r[1] += sf[j][1];
-      r[2] = fmax(r[2], sf[j][2]);
-      r[3] += sf[j][3];
-      for (int q2 = 0; q2 < NI; ++q2) ri[q2] += si[j][q2];
-    }
-    for (int q2 = 0; q2 < NF; ++q2) part_f[(long long)blockIdx.x * NF + q2] = r[q2];
-    for (int q2 = 0; q2 < NI; ++q2) part_i[(long long)blockIdx.x * (K + NI) + K + q2] = ri[q2];
-  }
-  for (int i = threadIdx.x; i < K; i += RB) part_i[(long long)blockIdx.x * (K + NI) + i] = hist[i];
-}
-
-// per-orientation column sums over fixed row chunks (sequential within a chunk)
-template <class TS>
-__global__ __launch_bounds__(256) void reduce_cols_kernel(const TS* __restrict__ eta, long long n, int K,
-                                                         long long nchunks, double* __restrict__ part_v) {
-  const long long tix = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (tix >= nchunks * K) return;
-  const long long ch = tix / K;
-  const int i = (int)(tix - ch * K);
-  const long long r0 = ch * kColRows, r1 = min(n, r0 + kColRows);
-  double s = 0.0;
-  for (long long r = r0; r < r1; ++r) s += (double)to_tc(eta[r * K + i]);
-  part_v[ch * K + i] = s;
-}
-
-__global__ __launch_bounds__(256) void reduce_final_kernel(int nb, long long nchunks, int K, double dV,
-                                                          const double* __restrict__ part_f,
-                                                          const long long* __restrict__ part_i,
-                                                          const double* __restrict__ part_v,
-                                                          double* __restrict__ out_f, long long* __restrict__ out_i) {
-  // one thread per output value, sequential over partials (fixed order)
-  const int tid = threadIdx.x;
-  for (int q = tid; q < NF; q += blockDim.x) {
-    double r = q == 2 ? -INFINITY : 0.0;
-    for (int b = 0; b < nb; ++b) r = q == 2 ? fmax(r, part_f[(long long)b * NF + q]) : r + part_f[(long long)b * NF + q];
-    out_f[q] = (q == 0 || q == 1) ? r * dV : r;
-  }
-  for (int i = tid; i < K; i += blockDim.x) {
-    double s = 0.0;
-    for (long long ch = 0; ch < nchunks; ++ch) s += part_v[ch * K + i];
-    out_f[NF + i] = s * dV;
-  }
-  for (int q = tid; q < K + NI; q += blockDim.x) {
-    long long s = 0;
-    for (int b = 0; b < nb; ++b) s += part_i[(long long)b * (K + NI) + q];
-    out_i[q] = s;
-  }
-}
-
 // CFD coupling (coupled/example.py:31-42): T_pf[(z, y, x)] = r T_past[(x, y, z)] + (1 - r) T_future[(x, y, z)]
 template <class TT>
 __global__ __launch_bounds__(256) void cfd_temperature_kernel(const TT* __restrict__ past, const TT* __restrict__ fut,
@@ -655,152 +466,6 @@ int pf_voronoi(const double* seeds_dev, int32_t n_seeds, const int32_t* grain_or
       seeds_dev, n_seeds, grain_ori_dev, p->nz, p->ny, p->nx, p->h[0], p->h[1], p->h[2], out_dev);
   hipError_t err = hipGetLastError();
   return err == hipSuccess ? PF_OK : hip_fail(err, "pf_voronoi launch");
-}
-
-int pf_argmax(const void* eta_dev, int32_t dtype, int64_t n_cells, int32_t k, int32_t* out_dev, void* stream) {
-  if (!eta_dev || !out_dev) return fail(PF_E_ARG, "NULL buffer");
-  if (!valid_dtype(dtype)) return fail(PF_E_ARG, "bad dtype");
-  if (n_cells < 1 || k < 1) return fail(PF_E_ARG, "n_cells and k must be >= 1");
-  if (!grid_ok(n_cells, 1)) return fail(PF_E_ARG, "grid too large");
-  const dim3 g((unsigned)((n_cells + 255) / 256));
-  hipStream_t s = (hipStream_t)stream;
-  switch (dtype) {
-    case PF_F64: argmax_kernel<double><<<g, 256, 0, s>>>((const double*)eta_dev, n_cells, k, out_dev); break;
-    case PF_F32: argmax_kernel<float><<<g, 256, 0, s>>>((const float*)eta_dev, n_cells, k, out_dev); break;
-    case PF_BF16: argmax_kernel<bf16_t><<<g, 256, 0, s>>>((const bf16_t*)eta_dev, n_cells, k, out_dev); break;
-  }
-  hipError_t err = hipGetLastError();
-  return err == hipSuccess ? PF_OK : hip_fail(err, "pf_argmax launch");
-}
-
-size_t pf_reduce_workspace_bytes(int64_t n_cells, int32_t k) {
-  if (n_cells < 1 || k < 1) return 0;
-  const long long nb = reduce_blocks(n_cells);
-  const long long nch = (n_cells + kColRows - 1) / kColRows;
-  return (size_t)(nb * NF * 8 + nb * (k + NI) * 8 + nch * k * 8);
-}
-
-}  // extern "C"
-
-namespace {
-
-// Argument checks shared by pf_reduce and pf_reduce_noalloc (host only, no HIP call):
-// fills the instance description and the workspace size the reduction needs.
-int reduce_check(const void* eta_dev, int32_t dtype, const void* T_dev, const pf_params_t* p,
-                 const double* out_f64_dev, const int64_t* out_i64_dev, StepDev& a, size_t& need) {
-  if (!eta_dev || !out_f64_dev || !out_i64_dev) return fail(PF_E_ARG, "NULL buffer");
-  int rc = make_stepdev(p, dtype, T_dev, (const void*)1, 0, a);
-  if (rc) return rc;
-  if (p->num_oris > RMAXK) return fail(PF_E_UNSUPPORTED, "pf_reduce supports K <= 256");
-  const long long n = (long long)p->nz * p->ny * p->nx;
-  const long long nch = (n + kColRows - 1) / kColRows;
-  if (!grid_ok(nch * p->num_oris, 1)) return fail(PF_E_ARG, "grid too large");
-  need = pf_reduce_workspace_bytes(n, p->num_oris);
-  return PF_OK;
-}
-
-// The three reduction launches over a workspace of at least pf_reduce_workspace_bytes bytes.
-// Every partial result is written before it is read, so the workspace needs no clearing.
-int reduce_launch(const StepDev& a, const void* eta_dev, int32_t dtype, const int32_t* argmax0_dev,
-                  const pf_params_t* p, double t, double* out_f64_dev, int64_t* out_i64_dev, void* ws_dev,
-                  void* stream) {
-  const int K = p->num_oris;
-  const long long n = (long long)p->nz * p->ny * p->nx;
-  const int nb = reduce_blocks(n);
-  const long long per_block = (n + nb - 1) / nb;
-  const long long nch = (n + kColRows - 1) / kColRows;
-  double* part_f = (double*)ws_dev;
-  long long* part_i = (long long*)(part_f + (long long)nb * NF);
-  double* part_v = (double*)(part_i + (long long)nb * (K + NI));
-  hipStream_t s = (hipStream_t)stream;
-  const double hk = 0.5 * p->kappa_g * p->ad_hoc;
-  const dim3 gc((unsigned)((nch * K + 255) / 256));
-  switch (dtype) {
-    case PF_F64:
-      reduce_cells_kernel<double><<<nb, RB, 0, s>>>(a, (const double*)eta_dev, argmax0_dev, t, p->m_g, p->gamma,
-                                                     p->ad_hoc, hk, per_block, part_f, part_i);
-      reduce_cols_kernel<double><<<gc, 256, 0, s>>>((const double*)eta_dev, n, K, nch, part_v);
-      break;
-    case PF_F32:
-      reduce_cells_kernel<float><<<nb, RB, 0, s>>>(a, (const float*)eta_dev, argmax0_dev, t, p->m_g, p->gamma,
-                                                    p->ad_hoc, hk, per_block, part_f, part_i);
-      reduce_cols_kernel<float><<<gc, 256, 0, s>>>((const float*)eta_dev, n, K, nch, part_v);
-      break;
-    case PF_BF16:
-      reduce_cells_kernel<bf16_t><<<nb, RB, 0, s>>>(a, (const bf16_t*)eta_dev, argmax0_dev, t, p->m_g, p->gamma,
-                                                     p->ad_hoc, hk, per_block, part_f, part_i);
-      reduce_cols_kernel<bf16_t><<<gc, 256, 0, s>>>((const bf16_t*)eta_dev, n, K, nch, part_v);
-      break;
-  }
-  const double dV = p->h[0] * p->h[1] * p->h[2];
-  reduce_final_kernel<<<1, 256, 0, s>>>(nb, nch, K, dV, part_f, part_i, part_v, out_f64_dev, (long long*)out_i64_dev);
-  hipError_t err = hipGetLastError();
-  return err == hipSuccess ? PF_OK : hip_fail(err, "pf_reduce launch");
-}
-
-}  // namespace
-
-// ---- allocation-free diagnostics (pf_reduce_noalloc)
-// The reduction's partial results live in this fixed array instead of a caller workspace.
-// Each GPU holds its own copy from code-object load until the process ends.  In host code
-// `scratch` names a host-side stand-in, not device memory: kernels get the device address
-// that hipGetSymbolAddress returns for the current device (scratch_dev below).
-static __device__ __align__(256) unsigned char scratch[PF_REDUCE_SCRATCH_BYTES];
-
-namespace {
-
-constexpr int kMaxDevices = 64;
-std::mutex g_scratch_mu;
-void* g_scratch_dev[kMaxDevices];  // device address of `scratch` per device, looked up once
-
-// Device address of `scratch` on the current device (set up on the first call per device).
-int scratch_dev(void** out) {
-  int dev = -1;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
-  if (dev < 0 || dev >= kMaxDevices) return fail(PF_E_UNSUPPORTED, "pf_reduce_noalloc supports devices 0..63");
-  std::lock_guard<std::mutex> lk(g_scratch_mu);
-  if (!g_scratch_dev[dev]) {
-    void* ptr = nullptr;
-    e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-    if (e != hipSuccess) return hip_fail(e, "hipGetSymbolAddress(scratch)");
-    if (!ptr) return fail(PF_E_HIP, "hipGetSymbolAddress(scratch) returned NULL");
-    g_scratch_dev[dev] = ptr;
-  }
-  *out = g_scratch_dev[dev];
-  return PF_OK;
-}
-
-}  // namespace
-
-extern "C" {
-
-int pf_reduce(const void* eta_dev, int32_t dtype, const void* T_dev, const int32_t* argmax0_dev,
-              const pf_params_t* p, double t, double* out_f64_dev, int64_t* out_i64_dev, void* ws_dev,
-              size_t ws_bytes, void* stream) {
-  StepDev a;
-  size_t need = 0;
-  int rc = reduce_check(eta_dev, dtype, T_dev, p, out_f64_dev, out_i64_dev, a, need);
-  if (rc) return rc;
-  if (!ws_dev) return fail(PF_E_ARG, "NULL workspace");
-  if (ws_bytes < need) return fail(PF_E_ARG, "workspace too small");
-  return reduce_launch(a, eta_dev, dtype, argmax0_dev, p, t, out_f64_dev, out_i64_dev, ws_dev, stream);
-}
-
-int pf_reduce_noalloc(const void* eta_dev, int32_t dtype, const void* T_dev, const int32_t* argmax0_dev,
-                      const pf_params_t* p, double t, double* out_f64_dev, int64_t* out_i64_dev, void* stream) {
-  StepDev a;
-  size_t need = 0;
-  int rc = reduce_check(eta_dev, dtype, T_dev, p, out_f64_dev, out_i64_dev, a, need);
-  if (rc) return rc;
-  if (need > (size_t)PF_REDUCE_SCRATCH_BYTES)
-    return fail(PF_E_ARG, "pf_reduce_noalloc: the reduction needs " + std::to_string(need) +
-                              " bytes of scratch, more than its fixed " + std::to_string(PF_REDUCE_SCRATCH_BYTES) +
-                              " (use pf_reduce with a workspace)");
-  void* ws = nullptr;
-  rc = scratch_dev(&ws);
-  if (rc) return rc;
-  return reduce_launch(a, eta_dev, dtype, argmax0_dev, p, t, out_f64_dev, out_i64_dev, ws, stream);
 }
 
 }  // extern "C"
