@@ -118,7 +118,7 @@ int pf_device_count(void);
  *   axes_dev: unique_grain_directions [3, K, 3] (utils.py:104-109), F64 when dtype == PF_F64 and F32
  *             otherwise; required when p->anisotropy > 0, else may be NULL.
  *   tile: index of the tile shape (pf_tile_count/pf_tile_shape), -1 for the default, or -2 to
- *         force the generic-K kernel (same arithmetic, one thread per cell, no LDS tiling).
+ *         force the generic-K kernel (same arithmetic, K at run time, no tiles in LDS).
  *   zchunk: z-planes per workgroup march (0 = default), optionally ORed with PF_ZCHUNK_TAIL.
  */
 int pf_step(const void* eta_in_dev, void* eta_out_dev, int32_t dtype, const void* T_dev,

@@ -202,33 +202,6 @@ void set_tiles(StepDev& a, int tx, int ty, int zchunk) {
   a.tiles_z = (a.zsplit > 0 ? (a.zsplit + a.zs - 1) / a.zs : 0) + (a.nz - a.zsplit + zc - 1) / zc;
 }
 
-StepLaunch generic_step(int dtype, bool aniso) {
-  switch (dtype) {
-    case PF_F64: return aniso ? &launch_generic<double, true> : &launch_generic<double, false>;
-    case PF_F32: return aniso ? &launch_generic<float, true> : &launch_generic<float, false>;
-    case PF_BF16: return aniso ? &launch_generic<bf16_t, true> : &launch_generic<bf16_t, false>;
-  }
-  return nullptr;
-}
-
-static StepLaunch generic_rhs(int dtype, bool aniso) {
-  switch (dtype) {
-    case PF_F64: return aniso ? &launch_generic<double, true, true> : &launch_generic<double, false, true>;
-    case PF_F32: return aniso ? &launch_generic<float, true, true> : &launch_generic<float, false, true>;
-    case PF_BF16: return aniso ? &launch_generic<bf16_t, true, true> : &launch_generic<bf16_t, false, true>;
-  }
-  return nullptr;
-}
-
-BatchLaunch generic_batch(int dtype, bool aniso) {
-  switch (dtype) {
-    case PF_F64: return aniso ? &launch_batch_generic<double, true> : &launch_batch_generic<double, false>;
-    case PF_F32: return aniso ? &launch_batch_generic<float, true> : &launch_batch_generic<float, false>;
-    case PF_BF16: return aniso ? &launch_batch_generic<bf16_t, true> : &launch_batch_generic<bf16_t, false>;
-  }
-  return nullptr;
-}
-
 // ------------------------------------------------------------------ auxiliary kernels
 template <class TT>
 __global__ __launch_bounds__(256) void temperature_kernel(const StepDev a, TT* __restrict__ out, double t) {
@@ -379,7 +352,8 @@ int pf_step(const void* eta_in_dev, void* eta_out_dev, int32_t dtype, const void
     if (tile > 0 && entry_count(dtype, p->num_oris, aniso) > 0) return fail(PF_E_ARG, "no such tile shape");
     const long long n = (long long)p->nz * p->ny * p->nx;
     if (!grid_ok(n, 1)) return fail(PF_E_ARG, "grid too large for the generic kernel");
-    err = generic_step(dtype, aniso)(a, d, (hipStream_t)stream);
+    set_quads(a, dtype, zchunk > 0 && zchunk <= 0xffff ? zchunk : 0);
+    err = generic_step(dtype, p->num_oris, aniso)(a, d, (hipStream_t)stream);
   }
   if (err != hipSuccess) return hip_fail(err, "pf_step launch");
   return PF_OK;
@@ -395,7 +369,8 @@ int pf_rhs(const void* eta_in_dev, void* rhs_out_dev, int32_t dtype, const void*
   const StepDyn d = make_dyn(a, eta_in_dev, rhs_out_dev, t, 1.0);  // c1, c2 carry L only: rhs = -L (grad + laplace)
   const long long n = (long long)p->nz * p->ny * p->nx;
   if (!grid_ok(n, 1)) return fail(PF_E_ARG, "grid too large");
-  hipError_t err = generic_rhs(dtype, p->anisotropy > 0.0)(a, d, (hipStream_t)stream);
+  set_quads(a, dtype, 0);
+  hipError_t err = generic_rhs(dtype, p->num_oris, p->anisotropy > 0.0)(a, d, (hipStream_t)stream);
   return err == hipSuccess ? PF_OK : hip_fail(err, "pf_rhs launch");
 }
 

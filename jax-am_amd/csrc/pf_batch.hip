@@ -66,7 +66,8 @@ struct BatchClass {
 struct SlotHost {
   bool used = false;
   int cls = -1;
-  int items = 0;  // work items of this slot
+  int items = 0;   // work items of this slot
+  int charge = 0;  // what the slot counts for against max_tiles
 };
 
 }  // namespace pf
@@ -81,6 +82,7 @@ struct pf_batch {
   StepDyn* d_dyn = nullptr;
   BatchSlot* d_slots = nullptr;
   WorkItem* d_work = nullptr;
+  size_t work_cap = 0;     // items that d_work holds (at least max_tiles)
   int2* d_info = nullptr;  // per class (work-list offset, count)
   std::vector<SlotHost> slots;
   std::vector<BatchClass> classes;
@@ -98,6 +100,14 @@ struct pf_batch {
 
 namespace {
 
+void drop_graphs(pf_batch* b) {
+  for (pf_batch::Graph& g : b->graphs) {
+    (void)hipGraphExecDestroy(g.exec);
+    (void)hipGraphDestroy(g.def);
+  }
+  b->graphs.clear();
+}
+
 int rebuild_work(pf_batch* b) {
   // pack each class's work items contiguously, in slot order
   std::vector<std::vector<WorkItem>> per(b->classes.size());
@@ -114,8 +124,21 @@ int rebuild_work(pf_batch* b) {
     info[c] = make_int2((int)all.size(), (int)per[c].size());
     all.insert(all.end(), per[c].begin(), per[c].end());
   }
-  if ((int)all.size() > b->max_tiles) return fail(PF_E_ARG, "batch work list exceeds max_tiles");
   hipError_t e = hipSuccess;
+  if (all.size() > b->work_cap) {
+    // more items than max_tiles (slots are charged by the cells of a kernel of one thread per cell):
+    // a longer list; the graphs that hold the old one's address go with it
+    WorkItem* grown = nullptr;
+    const size_t cap = all.size() + all.size() / 2;
+    e = hipMalloc((void**)&grown, sizeof(WorkItem) * cap);
+    if (e != hipSuccess) return hip_fail(e, "pf_batch work list");
+    e = hipStreamSynchronize(b->stream);
+    drop_graphs(b);
+    (void)hipFree(b->d_work);
+    b->d_work = grown;
+    b->work_cap = cap;
+    if (e != hipSuccess) return hip_fail(e, "pf_batch work list");
+  }
   if (!all.empty())
     e = hipMemcpyAsync(b->d_work, all.data(), all.size() * sizeof(WorkItem), hipMemcpyHostToDevice, b->stream);
   if (e == hipSuccess)
@@ -138,20 +161,12 @@ int launch_step_all(pf_batch* b) {
   for (size_t c = 0; c < b->classes.size(); ++c) {
     const BatchClass& k = b->classes[c];
     if (k.count == 0) continue;
-    hipError_t e = k.fn(b->d_desc, b->d_dyn, b->d_slots, b->d_work, b->d_info, (int)c, k.grid, b->stream);
+    hipError_t e = k.fn(b->d_desc, b->d_dyn, b->d_slots, b->d_work, b->d_info, (int)c, k.grid, k.k, b->stream);
     if (e != hipSuccess) return hip_fail(e, "pf_batch step launch");
   }
   advance_kernel<<<(b->max_inst + 63) / 64, 64, 0, b->stream>>>(b->d_desc, b->d_slots, b->d_dyn, b->max_inst);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? PF_OK : hip_fail(e, "pf_batch advance launch");
-}
-
-void drop_graphs(pf_batch* b) {
-  for (pf_batch::Graph& g : b->graphs) {
-    (void)hipGraphExecDestroy(g.exec);
-    (void)hipGraphDestroy(g.def);
-  }
-  b->graphs.clear();
 }
 
 // Destroy the cached graphs that launch class c (its index is about to be retired).  The
@@ -223,6 +238,7 @@ pf_batch_t* pf_batch_create(int32_t max_instances, int32_t max_tiles, void* stre
   b->max_inst = max_instances;
   b->max_tiles = max_tiles;
   b->stream = (hipStream_t)stream;
+  b->work_cap = max_tiles;
   b->slots.resize(max_instances);
   hipError_t e = hipMalloc((void**)&b->d_desc, sizeof(StepDev) * max_instances);
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_dyn, sizeof(StepDyn) * max_instances);
@@ -282,28 +298,30 @@ int pf_batch_add(pf_batch_t* b, const pf_batch_inst_t* inst) {
   if (rc) return rc;
   const bool aniso = inst->p.anisotropy > 0.0;
   const StepEntry* e = find_entry(inst->dtype, inst->p.num_oris, aniso, inst->tile);
-  int items, tile = -1, grid;
+  int items, charge, tile = -1, grid;
   BatchLaunch fn;
   if (e) {
     if (march_fits(&inst->p, inst->dtype)) return PF_E_ARG;
     set_tiles(a, e->tx, e->ty, inst->zchunk);
-    items = a.tiles_x * a.tiles_y * a.tiles_z;
+    items = charge = a.tiles_x * a.tiles_y * a.tiles_z;
     tile = e->tile;
     fn = e->batch;
     grid = 1024;
   } else {
     if (inst->tile > 0 && entry_count(inst->dtype, inst->p.num_oris, aniso) > 0)
       return fail(PF_E_ARG, "no such tile shape");
-    const long long n = (long long)inst->p.nz * inst->p.ny * inst->p.nx;
-    if ((n + 255) / 256 >= (1LL << 31)) return fail(PF_E_ARG, "instance too large");
-    items = (int)((n + 255) / 256);
-    fn = generic_batch(inst->dtype, aniso);
+    const long long n = set_quads(a, inst->dtype, 0);
+    if (n >= (1LL << 31) || ((long long)inst->p.nz * inst->p.ny * inst->p.nx + 255) / 256 >= (1LL << 31))
+      return fail(PF_E_ARG, "instance too large");
+    items = (int)n;
+    charge = (int)(((long long)inst->p.nz * inst->p.ny * inst->p.nx + 255) / 256);
+    fn = generic_batch(inst->dtype, inst->p.num_oris, aniso);
     grid = 2048;
   }
   int total = 0;
   for (const SlotHost& sh : b->slots)
-    if (sh.used) total += sh.items;
-  if (total + items > b->max_tiles) return fail(PF_E_STATE, "batch work list full (max_tiles)");
+    if (sh.used) total += sh.charge;
+  if (total + charge > b->max_tiles) return fail(PF_E_STATE, "batch work list full (max_tiles)");
   int cls = -1, free_cls = -1;
   for (size_t c = 0; c < b->classes.size(); ++c) {
     const BatchClass& k = b->classes[c];
@@ -357,6 +375,7 @@ int pf_batch_add(pf_batch_t* b, const pf_batch_inst_t* inst) {
   b->slots[slot].used = true;
   b->slots[slot].cls = cls;
   b->slots[slot].items = items;
+  b->slots[slot].charge = charge;
   b->classes[cls].users += 1;
   b->work_dirty = true;
   return slot;

@@ -1219,10 +1219,196 @@ __device__ __forceinline__ void march_tile(const StepDev& a, const StepDyn& d, i
   m.run();
 }
 
-// ------------------------------------------------------------------ generic-K march
-// One thread per cell, K at run time, neighbours straight from global memory.  Used for
-// K without a register-tiled instantiation.  Same per-cell and per-channel arithmetic
-// as march_tile.  RHS = true writes state_rhs instead of the Euler update.
+// ------------------------------------------------------------------ channel groups
+// Channels per thread for K channels: 16 bytes of FP32 or FP64, 8 bytes of BF16 (K is more often a
+// multiple of 4 than of 8), or the largest smaller power of two that K holds.
+template <class TS> constexpr int quad_cap() { return sizeof(TS) == 8 ? 2 : 4; }
+inline int quad_of(int dtype, int K) {
+  const int cap = dtype == PF_F64 ? 2 : 4;
+  return K >= cap ? cap : K >= 2 ? 2 : 1;
+}
+
+// A thread's channels [s, s + V) of its cell.  TAIL (K not a multiple of V): the last group of a cell
+// overlaps the one before it, s = min(V q, K - V), so that its load stays inside the cell; its
+// first e0 = V q - s channels are not its own and read as +0.
+template <class TS, int V, bool TAIL> struct QuadAt {
+  using TC = typename Traits<TS>::TC;
+  using BT = typename std::conditional<sizeof(TC) == 8, unsigned long long, unsigned>::type;
+  int s, e0;
+  __device__ __forceinline__ QuadAt(int K, int q) : s(TAIL ? min(V * q, K - V) : V * q), e0(TAIL ? V * q - s : 0) {}
+  using QV = VecA<TS, V, (int)sizeof(TS)>;
+  __device__ __forceinline__ QV raw(const TS* __restrict__ cell) const { return *(const QV*)(cell + s); }
+  __device__ __forceinline__ void load(const TS* __restrict__ cell, TC (&v)[V]) const {
+    const QV r = raw(cell);
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      v[e] = to_tc(r.v[e]);
+      if constexpr (TAIL) v[e] = __builtin_bit_cast(TC, __builtin_bit_cast(BT, v[e]) & (e >= e0 ? ~(BT)0 : (BT)0));
+    }
+  }
+};
+
+
+// ------------------------------------------------------------------ march of channel groups
+// Any K at run time.  The K channels of a cell are dealt to Q = ceil(K / V) threads of V consecutive
+// channels; a workgroup of kQuadT threads owns a run of C = kQuadT / Q cells of a z-plane (contiguous
+// memory) and marches it up through `zc` planes.  Each thread keeps its channels at z-1, z and z+1 in
+// registers and reads its x- and y-neighbours straight from global memory (the x-neighbours are in
+// lines that its wavefront has just read, the y-neighbours in lines of the same XCD's L2: quad_tile),
+// so that every access of a wavefront is a contiguous run whatever K is.  The centre values of
+// the run go through LDS once per plane, where every thread forms its cell's sum of squares in the
+// order of sum_sq_halves; the per-cell coefficients of the whole march are evaluated first, by all
+// threads, into an LDS table.  One barrier per plane.  Same per-cell and per-channel arithmetic as
+// the tiled march: results are bitwise the same.
+// 97x101x45, K = 33, FP32, anisotropic: 1336 us with one thread per cell (7 value-by-value strided
+// reads per channel), 46 us here (3.1e11 updates/s; reading and writing the state once takes 19 us);
+// pf_rhs on 96x80x40, K = 16, FP64: 415 us against 24 us.  Bound by its VALU work, about 90
+// instructions per channel: a wavefront's lanes hold different channels, so that a channel that is
+// zero everywhere can not be skipped as the tiled march does it (256x256x64, K = 20, FP32: 197 us
+// against 133 us there).
+// RHS = true writes state_rhs instead of the Euler update.
+constexpr int kQuadT = 256;
+constexpr int kQuadTab = 512;  // (cell, plane) pairs of a march at most
+
+template <class TC> struct QuadCoef {
+  TC c1, A0, w1, w2;  // CellCoef without S (A = 4 gamma S + A0); isotropic: w1 = c2
+};
+
+template <class TS, int V> struct QuadLds {
+  using TC = typename Traits<TS>::TC;
+  alignas(16) TC rows[2][kQuadT * V + 4];
+  alignas(16) QuadCoef<TC> coef[kQuadTab];
+  unsigned char liquid[kQuadTab];
+};
+
+// Run and layer of workgroup t: workgroups are dealt round-robin to the 8 XCDs; XCD x walks its own
+// eighth of the plane's runs, so that the rows above and below a run are in its own L2.  Layers go
+// from the top of the domain down (tile_coords).
+__device__ __forceinline__ bool quad_tile(const StepDev& a, int t, int& run, int& layer) {
+  const int m = a.tiles_y;  // runs per XCD
+  const int i = t >> 3, l = i / m;
+  layer = a.tiles_z - 1 - l;
+  run = (t & 7) * m + (i - l * m);
+  return run < a.tiles_x;
+}
+
+template <class TS, bool ANISO, bool RHS, int V, bool TAIL>
+__device__ __forceinline__ void quad_march(const StepDev& a, const StepDyn& d, int run, int layer,
+                                           QuadLds<TS, V>& lds, typename Traits<TS>::TC* __restrict__ ax) {
+  using TC = typename Traits<TS>::TC;
+  const int tid = threadIdx.x;
+  const int K = a.k, nx = a.nx, nxy = a.nx * a.ny;
+  const int Q = (K + V - 1) / V, C = kQuadT / Q;
+  const int zb = layer * a.zc, len = min(a.nz - zb, a.zc);
+  const int p0 = run * C;
+  const int j = tid / Q;
+  const QuadAt<TS, V, TAIL> at(K, tid - j * Q);
+  const int p = p0 + j;
+  const bool on = j < C && p < nxy;
+  const int py = p / nx, px = p - py * nx;
+  const long long plane = (long long)nxy * K;
+  const TS* r = (const TS*)d.in + zb * plane + (long long)p * K;
+  const int oxm = px > 0 ? -K : 0, oxp = px < nx - 1 ? K : 0;
+  const int oym = py > 0 ? -nx * K : 0, oyp = py < a.ny - 1 ? nx * K : 0;
+  // Groups are loaded whole: in the last group of a TAIL cell the channels before e0 are computed
+  // from the values of the group before it and not used.
+  using QV = typename QuadAt<TS, V, TAIL>::QV;
+  QV lo, c, n;
+  if (on) {
+    c = at.raw(r - (zb > 0 ? plane : 0));
+    n = at.raw(r);
+  }
+  if constexpr (ANISO) {
+    const TC* axes = (const TC*)a.axes;
+    for (int w = tid; w < 9 * K; w += kQuadT) {
+      const int i = w / 9, e = w - 9 * i;
+      const int k = e / 3, x = e - 3 * k;
+      ax[12 * i + 4 * k + x] = axes[(k * K + i) * 3 + x];
+    }
+  }
+  for (int i = tid; i < len * C; i += kQuadT) {
+    const int l = i / C, pc = p0 + (i - l * C);
+    if (pc < nxy) {
+      const int cy = pc / nx;
+      const CellCoef<TC> cf = cell_coef<TC>(a, d.cold, pc - cy * nx, cy, zb + l, (long long)(zb + l) * nxy + pc,
+                                            d.t_prev, d.hstep, (TC)0);
+      lds.coef[i] = QuadCoef<TC>{cf.c1, cf.A, ANISO ? cf.w1 : cf.c2, cf.w2};
+      lds.liquid[i] = cf.liquid;
+    }
+  }
+  const TC B = lap_B<TC>(a);
+  TC ihx2, ihy2, ihz2;
+  inv_h2<TC>(a, ihx2, ihy2, ihz2);
+  const TC g4 = (TC)a.gamma4;
+  const int h = K / 2;
+  TS* o = (TS*)d.out + zb * plane + (long long)p * K;
+  for (int l = 0; l < len; ++l) {
+    const int z = zb + l;
+    lo = c;
+    c = n;
+    TC* rows = lds.rows[l & 1];
+    QV xm, xp, ym, yp;
+    if (on) {
+      xm = at.raw(r + oxm);
+      xp = at.raw(r + oxp);
+      ym = at.raw(r + oym);
+      yp = at.raw(r + oyp);
+      n = at.raw(r + (z < a.nz - 1 ? plane : 0));  // the plane above the domain's last is that plane itself
+      TC* w = rows + j * (Q * V) + at.s;
+#pragma unroll
+      for (int e = 0; e < V; ++e)
+        if (!TAIL || e >= at.e0) w[e] = to_tc(c.v[e]);
+    }
+    lds_barrier();
+    if (on) {
+      const TC* row = rows + j * (Q * V);
+      TC s0 = 0, s1 = 0;
+#pragma unroll 4
+      for (int i = 0; i < h; ++i) {
+        s0 = fmac(row[i], row[i], s0);
+        s1 = fmac(row[h + i], row[h + i], s1);
+      }
+      if (K & 1) s1 = fmac(row[K - 1], row[K - 1], s1);
+      const int ci = l * C + j;
+      const QuadCoef<TC> q = lds.coef[ci];
+      CellCoef<TC> cf;
+      cf.c1 = q.c1;
+      cf.c2 = cf.w1 = q.w1;
+      cf.w2 = q.w2;
+      cf.A = fmac(g4, sum_sq_halves(s0, s1), q.A0);
+      cf.liquid = !RHS && lds.liquid[ci];
+      const uint32_t key = sr_cell_key(sr_plane_key(d.seed, z), p) + (uint32_t)at.s * kSrChannel;
+      QV res;
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        const TC* axe = ax + 12 * (at.s + e);
+        const TC ce = to_tc(c.v[e]), x0 = to_tc(xm.v[e]), x1 = to_tc(xp.v[e]), y0 = to_tc(ym.v[e]),
+                 y1 = to_tc(yp.v[e]), z0 = to_tc(lo.v[e]), z1 = to_tc(n.v[e]);
+        TC v;
+        if constexpr (RHS)
+          v = update_one<TC, ANISO, true>(cf, B, ihx2, ihy2, ihz2, ce, x0, x1, y0, y1, z0, z1, axe);
+        else
+          v = update_sr<TS, ANISO>(cf, B, ihx2, ihy2, ihz2, ce, x0, x1, y0, y1, z0, z1, axe,
+                                   key + (uint32_t)e * kSrChannel);
+        res.v[e] = from_tc<TS>(cf.liquid ? (TC)0 : v);
+      }
+      if (!TAIL || at.e0 == 0) {
+        *(QV*)(o + at.s) = res;
+      } else {
+#pragma unroll
+        for (int e = 1; e < V; ++e)
+          if (e >= at.e0) o[at.s + e] = res.v[e];
+      }
+    }
+    r += plane;
+    o += plane;
+  }
+}
+
+// ------------------------------------------------------------------ one thread per cell
+// K at run time, neighbours straight from global memory: K of more channels than the groups of one
+// workgroup hold.  Same per-cell and per-channel arithmetic as march_tile.  RHS = true writes
+// state_rhs instead of the Euler update.
 template <class TS, bool ANISO, bool RHS = false>
 __device__ __forceinline__ void generic_cell(const StepDev& a, const StepDyn& dy, long long cell) {
   using TC = typename Traits<TS>::TC;

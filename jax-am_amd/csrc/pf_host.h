@@ -3,6 +3,7 @@
 #pragma once
 
 #include <string>
+#include <type_traits>
 
 #include "pf_kernels.h"
 
@@ -30,5 +31,18 @@ int default_zchunk(int nz, int ny, int nx, int tx, int ty);
 // fills the tile grid (tiles_x/y/z, zc) for a tile shape
 int march_fits(const pf_params_t* p, int dtype);
 void set_tiles(StepDev& a, int tx, int ty, int zc);
+
+// f(V, TAIL) with the group size V as a constant
+template <class TS, class F>
+void with_quad(int K, int V, const F& f) {
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using IC = std::integral_constant<int, quad_cap<TS>()>;
+  if (V == 1) f(I1(), std::false_type());
+  else if (V != quad_cap<TS>() && K % 2 == 0) f(I2(), std::false_type());
+  else if (V != quad_cap<TS>()) f(I2(), std::true_type());
+  else if (K % V == 0) f(IC(), std::false_type());
+  else f(IC(), std::true_type());
+}
 
 }  // namespace pf

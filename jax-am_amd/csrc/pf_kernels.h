@@ -67,13 +67,6 @@ __global__ __launch_bounds__(TX* TY* H) __attribute__((amdgpu_waves_per_eu(H + 1
   march_tile<K, TS, ANISO, TX, TY, H>(a, d, tx, ty, tz, smem, stage, ax, &zt);
 }
 
-template <class TS, bool ANISO, bool RHS = false>
-__global__ __launch_bounds__(256) void generic_kernel(const StepDev a, const StepDyn d) {
-  const long long n = (long long)a.nz * a.ny * a.nx;
-  const long long cell = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (cell < n) generic_cell<TS, ANISO, RHS>(a, d, cell);
-}
-
 // Persistent batched step: a fixed grid walks the device-resident work list (slot,
 // tile) of one (dtype, K, anisotropy, tile shape) class.  Every workgroup exits after
 // the list is exhausted; slots with no steps left are skipped.  descs[slot] and
@@ -102,29 +95,9 @@ __global__ __launch_bounds__(TX* TY* H) __attribute__((amdgpu_waves_per_eu(2))) 
   }
 }
 
-// Batched generic-K step: work items are (slot, block of 256 cells).
-template <class TS, bool ANISO>
-__global__ __launch_bounds__(256) void batch_generic_kernel(const StepDev* __restrict__ descs,
-                                                           const StepDyn* __restrict__ dyns,
-                                                           const BatchSlot* __restrict__ slots,
-                                                           const WorkItem* __restrict__ work_all,
-                                                           const int2* __restrict__ cinfo, int cls) {
-  const int2 ci = cinfo[cls];
-  const WorkItem* __restrict__ work = work_all + ci.x;
-  for (int w = blockIdx.x; w < ci.y; w += gridDim.x) {
-    const WorkItem it = work[w];
-    const BatchSlot& s = slots[it.slot];
-    if (s.steps_left <= 0 || !s.active) continue;
-    const StepDev& a = descs[it.slot];
-    const long long n = (long long)a.nz * a.ny * a.nx;
-    const long long cell = (long long)it.tile * 256 + threadIdx.x;
-    if (cell < n) generic_cell<TS, ANISO>(a, dyns[it.slot], cell);
-  }
-}
-
 using StepLaunch = hipError_t (*)(const StepDev&, const StepDyn&, hipStream_t);
 using BatchLaunch = hipError_t (*)(const StepDev*, const StepDyn*, const BatchSlot*, const WorkItem*, const int2*,
-                                   int cls, int grid, hipStream_t);
+                                   int cls, int grid, int k, hipStream_t);
 
 struct StepEntry {
   int dtype, k, aniso, tile, tx, ty, h;
@@ -142,22 +115,8 @@ hipError_t launch_step(const StepDev& a, const StepDyn& d, hipStream_t s) {
 
 template <int K, class TS, bool ANISO, int TX, int TY, int H>
 hipError_t launch_batch(const StepDev* a, const StepDyn* d, const BatchSlot* sl, const WorkItem* w, const int2* ci,
-                        int cls, int grid, hipStream_t s) {
+                        int cls, int grid, int, hipStream_t s) {
   batch_kernel<K, TS, ANISO, TX, TY, H><<<dim3(grid), dim3(TX * TY * H), 0, s>>>(a, d, sl, w, ci, cls);
-  return hipGetLastError();
-}
-
-template <class TS, bool ANISO, bool RHS = false>
-hipError_t launch_generic(const StepDev& a, const StepDyn& d, hipStream_t s) {
-  const long long n = (long long)a.nz * a.ny * a.nx;
-  generic_kernel<TS, ANISO, RHS><<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s>>>(a, d);
-  return hipGetLastError();
-}
-
-template <class TS, bool ANISO>
-hipError_t launch_batch_generic(const StepDev* a, const StepDyn* d, const BatchSlot* sl, const WorkItem* w,
-                                const int2* ci, int cls, int grid, hipStream_t s) {
-  batch_generic_kernel<TS, ANISO><<<dim3(grid), dim3(256), 0, s>>>(a, d, sl, w, ci, cls);
   return hipGetLastError();
 }
 
@@ -188,8 +147,12 @@ const StepEntry* step_table_part_8(int* n);
 const StepEntry* step_table_part_9(int* n);
 const StepEntry* step_table_part_10(int* n);
 const StepEntry* step_table_part_11(int* n);
-// generic-K launchers by dtype
-StepLaunch generic_step(int dtype, bool aniso);
-BatchLaunch generic_batch(int dtype, bool aniso);
+// Kernels for any K (pf_quad.hip): the march of channel groups, and one thread per cell for K of more
+// groups than a workgroup's threads.  set_quads fills a's tile fields for (dtype, K) and returns the
+// number of workgroups (work items of the batched kernel) of a launch.
+long long set_quads(StepDev& a, int dtype, int zc);
+StepLaunch generic_step(int dtype, int k, bool aniso);
+StepLaunch generic_rhs(int dtype, int k, bool aniso);
+BatchLaunch generic_batch(int dtype, int k, bool aniso);
 
 }  // namespace pf

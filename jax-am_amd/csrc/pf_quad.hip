@@ -1,0 +1,165 @@
+// Step and right-hand-side kernels for any K: the march of channel groups (pf_device.h quad_march),
+// and one thread per cell for K of more groups than a workgroup has threads.
+#include "pf_host.h"
+
+namespace pf {
+
+template <class TS, bool ANISO, bool RHS, int V, bool TAIL>
+__global__ __launch_bounds__(kQuadT) void quad_kernel(const StepDev a, const StepDyn d) {
+  __shared__ QuadLds<TS, V> lds;
+  extern __shared__ __attribute__((aligned(16))) char axmem[];
+  int run, layer;
+  if (quad_tile(a, blockIdx.x, run, layer))
+    quad_march<TS, ANISO, RHS, V, TAIL>(a, d, run, layer, lds, (typename Traits<TS>::TC*)axmem);
+}
+
+// Batched: work items are (slot, workgroup of the slot's own launch).
+template <class TS, bool ANISO, int V, bool TAIL>
+__global__ __launch_bounds__(kQuadT) void batch_quad_kernel(const StepDev* __restrict__ descs,
+                                                           const StepDyn* __restrict__ dyns,
+                                                           const BatchSlot* __restrict__ slots,
+                                                           const WorkItem* __restrict__ work_all,
+                                                           const int2* __restrict__ cinfo, int cls) {
+  __shared__ QuadLds<TS, V> lds;
+  extern __shared__ __attribute__((aligned(16))) char axmem[];
+  const int2 ci = cinfo[cls];
+  const WorkItem* __restrict__ work = work_all + ci.x;
+  for (int w = blockIdx.x; w < ci.y; w += gridDim.x) {
+    const WorkItem it = work[w];
+    const BatchSlot& s = slots[it.slot];
+    if (s.steps_left <= 0 || !s.active) continue;
+    const StepDev& a = descs[it.slot];
+    int run, layer;
+    if (!quad_tile(a, it.tile, run, layer)) continue;
+    quad_march<TS, ANISO, false, V, TAIL>(a, dyns[it.slot], run, layer, lds, (typename Traits<TS>::TC*)axmem);
+    lds_barrier();  // LDS is reused by the next item
+  }
+}
+
+template <class TS, bool ANISO, bool RHS>
+__global__ __launch_bounds__(256) void generic_kernel(const StepDev a, const StepDyn d) {
+  const long long n = (long long)a.nz * a.ny * a.nx;
+  const long long cell = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (cell < n) generic_cell<TS, ANISO, RHS>(a, d, cell);
+}
+
+// Batched, one thread per cell: work items are (slot, block of 256 cells).
+template <class TS, bool ANISO>
+__global__ __launch_bounds__(256) void batch_generic_kernel(const StepDev* __restrict__ descs,
+                                                           const StepDyn* __restrict__ dyns,
+                                                           const BatchSlot* __restrict__ slots,
+                                                           const WorkItem* __restrict__ work_all,
+                                                           const int2* __restrict__ cinfo, int cls) {
+  const int2 ci = cinfo[cls];
+  const WorkItem* __restrict__ work = work_all + ci.x;
+  for (int w = blockIdx.x; w < ci.y; w += gridDim.x) {
+    const WorkItem it = work[w];
+    const BatchSlot& s = slots[it.slot];
+    if (s.steps_left <= 0 || !s.active) continue;
+    const StepDev& a = descs[it.slot];
+    const long long n = (long long)a.nz * a.ny * a.nx;
+    const long long cell = (long long)it.tile * 256 + threadIdx.x;
+    if (cell < n) generic_cell<TS, ANISO>(a, dyns[it.slot], cell);
+  }
+}
+
+// channels per thread: a full group where K holds one, else single channels
+static int quad_v(int dtype, int K) {
+  const int cap = dtype == PF_F64 ? 2 : 4;
+  return K >= cap ? cap : 1;
+}
+// at most half a workgroup's threads per cell: the axis table of an anisotropic K stays under 25 KB
+static bool quad_fits(int dtype, int K) {
+  const int V = quad_v(dtype, K);
+  return (K + V - 1) / V <= kQuadT / 2;
+}
+constexpr int kQuadBlocks = 2048;  // eight workgroups on each of 256 CUs
+
+static size_t ax_bytes(int k, int tc, bool aniso) { return aniso ? (size_t)12 * k * tc : 16; }
+
+long long set_quads(StepDev& a, int dtype, int zc) {
+  const long long nxy = (long long)a.nx * a.ny;
+  if (!quad_fits(dtype, a.k)) return (nxy * a.nz + 255) / 256;
+  const int V = quad_v(dtype, a.k), Q = (a.k + V - 1) / V, C = kQuadT / Q;
+  const long long runs = (nxy + C - 1) / C;
+  if (zc <= 0) {
+    // about kQuadBlocks workgroups (a plane more per march costs less than its two planes outside)
+    const long long chunks = (kQuadBlocks + runs - 1) / runs;
+    zc = (int)((a.nz + chunks - 1) / chunks);
+  }
+  if (zc > kQuadTab / C) zc = kQuadTab / C;
+  if (zc > a.nz) zc = a.nz;
+  a.zc = a.zs = zc;
+  a.zsplit = 0;
+  a.tiles_x = (int)runs;
+  a.tiles_y = (int)((runs + 7) / 8);
+  a.tiles_z = (a.nz + zc - 1) / zc;
+  return 8LL * a.tiles_y * a.tiles_z;
+}
+
+template <class TS, bool ANISO, bool RHS>
+static hipError_t launch_quad(const StepDev& a, const StepDyn& d, hipStream_t s) {
+  using TC = typename Traits<TS>::TC;
+  constexpr int dt = Traits<TS>::dtype;
+  const unsigned nb = 8u * a.tiles_y * a.tiles_z;
+  const size_t sh = ax_bytes(a.k, sizeof(TC), ANISO);
+  const int V = quad_v(dt, a.k);
+  if (V == 1) quad_kernel<TS, ANISO, RHS, 1, false><<<nb, kQuadT, sh, s>>>(a, d);
+  else if (a.k % V == 0) quad_kernel<TS, ANISO, RHS, quad_cap<TS>(), false><<<nb, kQuadT, sh, s>>>(a, d);
+  else quad_kernel<TS, ANISO, RHS, quad_cap<TS>(), true><<<nb, kQuadT, sh, s>>>(a, d);
+  return hipGetLastError();
+}
+
+template <class TS, bool ANISO, bool RHS>
+static hipError_t launch_cells(const StepDev& a, const StepDyn& d, hipStream_t s) {
+  const long long n = (long long)a.nz * a.ny * a.nx;
+  generic_kernel<TS, ANISO, RHS><<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s>>>(a, d);
+  return hipGetLastError();
+}
+
+template <class TS, bool ANISO, int V, bool TAIL>
+static hipError_t launch_batch_quad(const StepDev* a, const StepDyn* d, const BatchSlot* sl, const WorkItem* w,
+                                    const int2* ci, int cls, int grid, int k, hipStream_t s) {
+  batch_quad_kernel<TS, ANISO, V, TAIL>
+      <<<dim3(grid), dim3(kQuadT), ax_bytes(k, sizeof(typename Traits<TS>::TC), ANISO), s>>>(a, d, sl, w, ci, cls);
+  return hipGetLastError();
+}
+
+template <class TS, bool ANISO>
+static hipError_t launch_batch_cells(const StepDev* a, const StepDyn* d, const BatchSlot* sl, const WorkItem* w,
+                                     const int2* ci, int cls, int grid, int, hipStream_t s) {
+  batch_generic_kernel<TS, ANISO><<<dim3(grid), dim3(256), 0, s>>>(a, d, sl, w, ci, cls);
+  return hipGetLastError();
+}
+
+template <class TS, bool RHS> static StepLaunch pick(int k, bool aniso) {
+  if (quad_fits(Traits<TS>::dtype, k)) return aniso ? &launch_quad<TS, true, RHS> : &launch_quad<TS, false, RHS>;
+  return aniso ? &launch_cells<TS, true, RHS> : &launch_cells<TS, false, RHS>;
+}
+template <class TS, bool ANISO> static BatchLaunch pick_batch(int k) {
+  const int V = quad_v(Traits<TS>::dtype, k);
+  if (!quad_fits(Traits<TS>::dtype, k)) return &launch_batch_cells<TS, ANISO>;
+  if (V == 1) return &launch_batch_quad<TS, ANISO, 1, false>;
+  return k % V == 0 ? &launch_batch_quad<TS, ANISO, quad_cap<TS>(), false>
+                    : &launch_batch_quad<TS, ANISO, quad_cap<TS>(), true>;
+}
+
+StepLaunch generic_step(int dtype, int k, bool aniso) {
+  return dtype == PF_F64   ? pick<double, false>(k, aniso)
+         : dtype == PF_F32 ? pick<float, false>(k, aniso)
+                           : pick<bf16_t, false>(k, aniso);
+}
+StepLaunch generic_rhs(int dtype, int k, bool aniso) {
+  return dtype == PF_F64   ? pick<double, true>(k, aniso)
+         : dtype == PF_F32 ? pick<float, true>(k, aniso)
+                           : pick<bf16_t, true>(k, aniso);
+}
+BatchLaunch generic_batch(int dtype, int k, bool aniso) {
+  switch (dtype) {
+    case PF_F64: return aniso ? pick_batch<double, true>(k) : pick_batch<double, false>(k);
+    case PF_F32: return aniso ? pick_batch<float, true>(k) : pick_batch<float, false>(k);
+    default: return aniso ? pick_batch<bf16_t, true>(k) : pick_batch<bf16_t, false>(k);
+  }
+}
+
+}  // namespace pf

@@ -23,44 +23,22 @@ constexpr int RMAXK = 256;  // pf_reduce handles K <= RMAXK
 constexpr int NF = 4;       // F_local, F_grad, max T, sum eta
 constexpr int NI = 3;       // changed, liquid, nonfinite
 
-// Channels per thread for K channels: 16 bytes of FP32 or FP64, 8 bytes of BF16 (K is more often a
-// multiple of 4 than of 8), or the largest smaller power of two that K holds.
-template <class TS> constexpr int quad_cap() { return sizeof(TS) == 8 ? 2 : 4; }
-inline int quad_of(int dtype, int K) {
-  const int cap = dtype == PF_F64 ? 2 : 4;
-  return K >= cap ? cap : K >= 2 ? 2 : 1;
+// numpy.argmax semantics among a thread's own channels: first maximum; a NaN is the maximum (first
+// NaN wins).
+template <class TS, int V, bool TAIL>
+__device__ __forceinline__ void quad_argmax(const QuadAt<TS, V, TAIL>& at, const typename Traits<TS>::TC (&v)[V],
+                                            typename Traits<TS>::TC& best, int& bi) {
+  typename Traits<TS>::TC b = v[0];
+  int i = at.s;
+#pragma unroll
+  for (int e = 1; e < V; ++e) {
+    const bool take = ((b == b) & !(v[e] <= b) & (e > at.e0)) | (TAIL & (e == at.e0));
+    b = take ? v[e] : b;
+    i = take ? at.s + e : i;
+  }
+  best = b;
+  bi = i;
 }
-
-// A thread's channels [s, s + V) of its cell.  TAIL (K not a multiple of V): the last group of a cell
-// overlaps the one before it, s = min(V q, K - V), so that its load stays inside the cell; its
-// first e0 = V q - s channels are not its own and read as +0.
-template <class TS, int V, bool TAIL> struct QuadAt {
-  using TC = typename Traits<TS>::TC;
-  using BT = typename std::conditional<sizeof(TC) == 8, unsigned long long, unsigned>::type;
-  int s, e0;
-  __device__ __forceinline__ QuadAt(int K, int q) : s(TAIL ? min(V * q, K - V) : V * q), e0(TAIL ? V * q - s : 0) {}
-  __device__ __forceinline__ void load(const TS* __restrict__ cell, TC (&v)[V]) const {
-    const VecA<TS, V, (int)sizeof(TS)> r = *(const VecA<TS, V, (int)sizeof(TS)>*)(cell + s);
-#pragma unroll
-    for (int e = 0; e < V; ++e) {
-      v[e] = to_tc(r.v[e]);
-      if constexpr (TAIL) v[e] = __builtin_bit_cast(TC, __builtin_bit_cast(BT, v[e]) & (e >= e0 ? ~(BT)0 : (BT)0));
-    }
-  }
-  // numpy.argmax semantics among the own channels: first maximum; a NaN is the maximum (first NaN wins)
-  __device__ __forceinline__ void argmax(const TC (&v)[V], TC& best, int& bi) const {
-    TC b = v[0];
-    int i = s;
-#pragma unroll
-    for (int e = 1; e < V; ++e) {
-      const bool take = ((b == b) & !(v[e] <= b) & (e > e0)) | (TAIL & (e == e0));
-      b = take ? v[e] : b;
-      i = take ? s + e : i;
-    }
-    best = b;
-    bi = i;
-  }
-};
 
 // Best of a cell's groups in order of their channels.
 template <class TC>
@@ -99,7 +77,7 @@ __global__ __launch_bounds__(RB) void argmax_kernel(const TS* __restrict__ eta, 
 #pragma unroll
   for (int r = 0; r < AR; ++r) at.load(base + (long long)min(r * C, n - 1 - j) * K, v[r]);
 #pragma unroll
-  for (int r = 0; r < AR; ++r) at.argmax(v[r], mx[r][threadIdx.x], ix[r][threadIdx.x]);
+  for (int r = 0; r < AR; ++r) quad_argmax(at, v[r], mx[r][threadIdx.x], ix[r][threadIdx.x]);
   __syncthreads();
   for (int i = threadIdx.x; i < n; i += RB) {
     const int r = i / C, cj = i - r * C;
@@ -306,7 +284,7 @@ __global__ __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(4))) void re
           if (zb + l > 0) sq_diff(v, prev, gz);
           s2[k * RB + tid] = S;
           s4[k * RB + tid] = F;
-          at.argmax(v, mx[k * RB + tid], ix[k * RB + tid]);
+          quad_argmax(at, v, mx[k * RB + tid], ix[k * RB + tid]);
 #pragma unroll
           for (int e = 0; e < V; ++e) prev[e] = v[e];
         }
@@ -415,19 +393,6 @@ __global__ __launch_bounds__(RB) void reduce_final_kernel(int nb, int K, double 
       out_i[i] = r;
     }
   }
-}
-
-// f(V, TAIL) with the group size V as a constant
-template <class TS, class F>
-static void with_quad(int K, int V, const F& f) {
-  using I1 = std::integral_constant<int, 1>;
-  using I2 = std::integral_constant<int, 2>;
-  using IC = std::integral_constant<int, quad_cap<TS>()>;
-  if (V == 1) f(I1(), std::false_type());
-  else if (V != quad_cap<TS>() && K % 2 == 0) f(I2(), std::false_type());
-  else if (V != quad_cap<TS>()) f(I2(), std::true_type());
-  else if (K % V == 0) f(IC(), std::false_type());
-  else f(IC(), std::true_type());
 }
 
 template <class TS>

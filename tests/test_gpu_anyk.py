@@ -1,0 +1,54 @@
+"""GPU parity of the kernels for any K (pf_step without a tiled instantiation, pf_rhs): K around a
+thread's channel group, up to and past the largest K of one workgroup, on grids whose planes are not
+whole runs of cells and whose planes are not whole marches."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import pf_oracle as O
+from pfkit import PFSolver
+from problems import args, gaussian, poly, quench
+
+pytestmark = pytest.mark.gpu
+
+# K: single channels, tails of every length, whole groups, the last K of the channel-group march in
+# FP64 (256) and FP32 (512) and the first past them
+CASES = [(7, 5, 9, 1), (19, 7, 3, 3), (23, 9, 40, 25), (11, 13, 5, 26), (10, 6, 9, 27), (16, 8, 21, 28), (29, 31, 7, 33),
+         (1, 1, 30, 40), (37, 1, 1, 64), (5, 4, 3, 256), (4, 3, 3, 257), (3, 3, 2, 512), (3, 2, 2, 513)]
+
+
+@pytest.mark.parametrize("nx,ny,nz,k", CASES)
+@pytest.mark.parametrize("aniso", [0.0, 0.15])
+def test_step_and_rhs_any_k(cuda, nx, ny, nz, k, aniso):
+    a = args(nx, ny, nz, k, anisotropy=aniso, force_liquid=True)
+    pc = poly(nx, ny, nz, k)
+    n = nx * ny * nz
+    rng = np.random.default_rng(n + k)
+    eta = np.where(rng.random((n, k)) < 0.3, 0.0, rng.random((n, k)))
+    cent = O.centroids(nz, ny, nx, pc.mesh_h_xyz)
+    for L in (gaussian(nx, ny, nz), quench(nz)):
+        T = O.laser_T(L.as_dict(), cent, 0.1)
+        # FP64: rounding of sums of up to k squares; FP32 storage: inputs rounded alike, one stochastic
+        # rounding (2^-23) of the result and FP32 sums of k terms of one sign, k 2^-24 of the sum S <= k
+        for dtype, tol in ((torch.float64, 1e-12), (torch.float32, 2e-6)):
+            e = torch.as_tensor(eta, dtype=dtype, device=cuda)
+            ed = e.double().cpu().numpy()
+            s = PFSolver(a, pc, dtype=dtype, device=cuda, clean=False, tile=-2, zchunk=0)
+            (out, _), _ = s.stepper((e, 0.1), 0.1001, [L])
+            ref = O.explicit_euler(ed, 0.1, 0.1001, T, a, pc.mesh_h_xyz, pc.unique_grain_directions)
+            assert np.max(np.abs(out.double().cpu().numpy() - ref)) <= tol * max(1.0, np.max(np.abs(ref)))
+            rhs = s.state_rhs(e, 0.1, [L]).double().cpu().numpy()
+            want = O.state_rhs(ed, T, a, pc.mesh_h_xyz, pc.unique_grain_directions)
+            assert np.max(np.abs(rhs - want)) <= max(tol, k * (6e-8 if dtype == torch.float32 else 0)) * max(1.0, np.max(np.abs(want)))
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("k", [3, 9, 10, 17, 20])
+def test_rhs_reads_unaligned_states(cuda, dtype, k):
+    nx, ny, nz = 21, 10, 7
+    a = args(nx, ny, nz, k, anisotropy=0.15)
+    s = PFSolver(a, poly(nx, ny, nz, k), dtype=dtype, device=cuda, clean=False)
+    n = nx * ny * nz
+    buf = torch.rand(n * k + 1, device=cuda, generator=torch.Generator(cuda).manual_seed(k)).to(dtype)
+    e = buf[1:].view(n, k)
+    assert torch.equal(s.state_rhs(e, 0.1, [gaussian(nx, ny, nz)]), s.state_rhs(e.clone(), 0.1, [gaussian(nx, ny, nz)]))
