@@ -117,7 +117,7 @@ int pf_device_count(void);
  *   T_dev: [N] temperature in p->laser.T_dtype when p->laser.model == PF_T_BUFFER, else ignored (may be NULL).
  *   axes_dev: unique_grain_directions [3, K, 3] (utils.py:104-109), F64 when dtype == PF_F64 and F32
  *             otherwise; required when p->anisotropy > 0, else may be NULL.
- *   tile: index of the tile shape (pf_tile_count/pf_tile_shape), -1 for the default, or -2 to
+ *   tile: index of the tile shape (pf_tile_count/pf_tile_shape), -1 for the library's choice (by size, K and dtype), or -2 to
  *         force the generic-K kernel (same arithmetic, K at run time, no tiles in LDS).
  *   zchunk: z-planes per workgroup march (0 = default), optionally ORed with PF_ZCHUNK_TAIL.
  */

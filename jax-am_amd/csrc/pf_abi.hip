@@ -4,6 +4,8 @@
 #include <math.h>
 #include <string.h>
 
+#include <atomic>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -122,6 +124,7 @@ int make_stepdev(const pf_params_t* p, int dtype, const void* T_dev, const void*
 namespace {
 struct Tables {
   std::vector<StepEntry> t[3];
+  std::unique_ptr<std::atomic<int>[]> held[3];  // per entry: workgroups the GPU holds at once (0: not asked yet)
   Tables() {
     using PartFn = const StepEntry* (*)(int*);
     const PartFn parts[kInstParts] = {&step_table_part_0, &step_table_part_1, &step_table_part_2,
@@ -133,6 +136,7 @@ struct Tables {
       const StepEntry* e = f(&n);
       for (int i = 0; i < n; ++i) t[e[i].dtype].push_back(e[i]);
     }
+    for (int d = 0; d < 3; ++d) held[d] = std::make_unique<std::atomic<int>[]>(t[d].size());
   }
 };
 const Tables& tables() {
@@ -157,6 +161,65 @@ const StepEntry* find_entry(int dtype, int k, bool aniso, int tile) {
   for (const StepEntry& e : tb.t[dtype])
     if (e.k == k && (e.aniso != 0) == aniso && e.tile == tile) return &e;
   return nullptr;
+}
+
+// Workgroups of e's step kernel that the GPU holds at once (asked of the runtime once per kernel).
+static int held_workgroups(const StepEntry* e) {
+  const Tables& tb = tables();
+  std::atomic<int>& c = tb.held[e->dtype][e - tb.t[e->dtype].data()];
+  int n = c.load(std::memory_order_relaxed);
+  if (n == 0) {
+    int per = 0, dev = 0, cus = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, e->kernel, e->tx * e->ty * e->h, 0) != hipSuccess ||
+        hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+      (void)hipGetLastError();
+      return 1024;
+    }
+    n = per * cus;
+    if (n < 1) n = 1;
+    c.store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
+// Planes per march for `cols` tile columns when the GPU holds `held` workgroups: the shortest marches
+// that fill it a whole number of times, once if they then have at most 12 planes, else as often as
+// that takes.  Each march reads two planes more than it writes, so longer is better, but only while
+// no CU idles at the launch's end: 128x96x48, K = 20, FP64 (16x4 lane pairs) 46.6 us at 12 planes, one
+// filling, against 51.4 at 6; 203x197x59, K = 17, FP32 (16x8) 87.7 us at 10, two fillings, against 91.4 at 8
+// and 100.3 at 16.
+static int fill_zchunk(int nz, long long cols, int held) {
+  const long long kmin = (nz + 11) / 12;
+  const long long m = (kmin * cols + held - 1) / held;  // fillings: the fewest whose chunks have at most 12 planes
+  const long long k = m * held / cols;
+  const long long zc = (nz + k - 1) / k;
+  return (int)(zc < 2 ? (nz < 2 ? nz : 2) : zc);
+}
+
+// The kernel of a step whose caller leaves the choice open, for K with tiled kernels: a tile shape,
+// or nullptr for the march of channel groups.  That one has a workgroup for every few hundred
+// cells and no LDS planes to fill first, which wins while the grid leaves the tiled kernels short of
+// workgroups, and for odd K in FP64, where a tile has one lane per cell and its registers spill; in
+// larger grids the tiles' exact skips of all-zero channels win.  Measured in us, groups against the best
+// tile (its best z-chunk): FP32 K = 10: 32^3 5.7/7.1, 64x64x32 8.7/8.3, 64^3 12.8/10.5; K = 20: 48x48x40 8.9/10.4,
+// 64x64x32 11.5/10.0; K = 17: 64x64x32 11.3/11.3, 64^3 17.5/14.2.  BF16 K = 20: 48x48x40 8.3/9.1; K = 10: 7.5/6.9;
+// K = 13: 64x64x32 9.1/9.3.  FP64 K = 10: 64x64x32 11.5/10.7 (isotropic 9.2/8.9), 48x48x40 9.3/10.2; K = 16: 64x64x32
+// 13.7/14.3, 64^3 20.3/21.2; K = 13: 96x96x48 30.9/33.2, 128x96x48 43.1/41.2; K = 17: 128x96x48 54.4/54.2.
+static const StepEntry* choose_step(int dtype, int k, bool aniso, long long cells) {
+  const long long t = quad_threads(dtype, k, cells);
+  const bool odd = k % 2 != 0;
+  long long most;
+  if (dtype == PF_F64) most = odd && k >= 11 ? 4000000 : k >= 16 ? 1100000 : 500000;
+  else if (dtype == PF_F32) most = odd ? 530000 : 470000;
+  else most = odd || k >= 16 ? 480000 : 250000;
+  if (t <= most) return nullptr;
+  int tile;
+  if (dtype == PF_F64) tile = !odd ? 2 : k >= 17 ? 0 : 1;       // 16x4 lane pairs; 32x4; 16x4
+  else if (k % 4 == 0 && k >= (dtype == PF_F32 ? 16 : 12)) tile = 4;  // 8x8 lane pairs (16-byte LDS reads need K % 4 = 0)
+  else tile = 2;                                                // 16x8
+  const StepEntry* e = find_entry(dtype, k, aniso, tile);
+  return e ? e : find_entry(dtype, k, aniso, 0);
 }
 
 int default_zchunk(int nz, int ny, int nx, int tx, int ty) {
@@ -344,15 +407,21 @@ int pf_step(const void* eta_in_dev, void* eta_out_dev, int32_t dtype, const void
     if (zchunk < 0 || (zchunk & ~(PF_ZCHUNK_TAIL | 0xffff)) != 0)
       return fail(PF_E_ARG, "zchunk must be a plane count in [0, 65535], optionally | PF_ZCHUNK_TAIL");
     if (march_fits(p, dtype)) return PF_E_ARG;
+    if (tile == -1) e = choose_step(dtype, p->num_oris, aniso, (long long)p->nz * p->ny * p->nx);
+  } else if (tile > 0 && entry_count(dtype, p->num_oris, aniso) > 0) {
+    return fail(PF_E_ARG, "no such tile shape");
+  }
+  if (e) {
+    const long long cols = (long long)((p->nx + e->tx - 1) / e->tx) * ((p->ny + e->ty - 1) / e->ty);
+    if ((zchunk & 0xffff) == 0) zchunk |= fill_zchunk(p->nz, cols, held_workgroups(e));
     set_tiles(a, e->tx, e->ty, zchunk);
     const long long nt = (long long)a.tiles_x * a.tiles_y * a.tiles_z;
     if (nt >= (1LL << 31)) return fail(PF_E_ARG, "too many tiles");
     err = e->step(a, d, (hipStream_t)stream);
   } else {
-    if (tile > 0 && entry_count(dtype, p->num_oris, aniso) > 0) return fail(PF_E_ARG, "no such tile shape");
     const long long n = (long long)p->nz * p->ny * p->nx;
     if (!grid_ok(n, 1)) return fail(PF_E_ARG, "grid too large for the generic kernel");
-    set_quads(a, dtype, zchunk > 0 && zchunk <= 0xffff ? zchunk : 0);
+    set_quads(a, dtype, zchunk > 0 ? zchunk & 0xffff : 0);
     err = generic_step(dtype, p->num_oris, aniso)(a, d, (hipStream_t)stream);
   }
   if (err != hipSuccess) return hip_fail(err, "pf_step launch");

@@ -104,6 +104,7 @@ struct StepEntry {
   StepLaunch step;
   BatchLaunch batch;
   size_t lds;
+  const void* kernel;  // the step kernel (occupancy queries)
 };
 
 template <int K, class TS, bool ANISO, int TX, int TY, int H>
@@ -130,7 +131,8 @@ hipError_t launch_batch(const StepDev* a, const StepDyn* d, const BatchSlot* sl,
    H,                                                                            \
    &launch_step<K, TS, (A != 0), TX, TY, H>,                                     \
    &launch_batch<K, TS, (A != 0), TX, TY, H>,                                    \
-   Tile<TS, K, TX, TY, H>::LDS_BYTES}
+   Tile<TS, K, TX, TY, H>::LDS_BYTES,                                            \
+   (const void*)&step_kernel<K, TS, (A != 0), TX, TY, H>}
 
 // instantiation tables, one per compiled part of pf_inst.hip (see Makefile):
 // parts 0-3 F32, 4-7 BF16, 8-11 F64, each over a K range
@@ -149,8 +151,10 @@ const StepEntry* step_table_part_10(int* n);
 const StepEntry* step_table_part_11(int* n);
 // Kernels for any K (pf_quad.hip): the march of channel groups, and one thread per cell for K of more
 // groups than a workgroup's threads.  set_quads fills a's tile fields for (dtype, K) and returns the
-// number of workgroups (work items of the batched kernel) of a launch.
+// number of workgroups (work items of the batched kernel) of a launch; quad_threads is the number
+// of its threads' channel groups in one pass over the grid.
 long long set_quads(StepDev& a, int dtype, int zc);
+long long quad_threads(int dtype, int k, long long cells);
 StepLaunch generic_step(int dtype, int k, bool aniso);
 StepLaunch generic_rhs(int dtype, int k, bool aniso);
 BatchLaunch generic_batch(int dtype, int k, bool aniso);

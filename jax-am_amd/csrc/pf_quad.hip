@@ -73,9 +73,14 @@ static bool quad_fits(int dtype, int K) {
   const int V = quad_v(dtype, K);
   return (K + V - 1) / V <= kQuadT / 2;
 }
-constexpr int kQuadBlocks = 2048;  // eight workgroups on each of 256 CUs
+constexpr int kQuadBlocks = 1280;  // five workgroups on each of 256 CUs (what the registers allow)
 
 static size_t ax_bytes(int k, int tc, bool aniso) { return aniso ? (size_t)12 * k * tc : 16; }
+
+long long quad_threads(int dtype, int k, long long cells) {
+  const int V = quad_v(dtype, k);
+  return cells * ((k + V - 1) / V);
+}
 
 long long set_quads(StepDev& a, int dtype, int zc) {
   const long long nxy = (long long)a.nx * a.ny;
@@ -83,8 +88,8 @@ long long set_quads(StepDev& a, int dtype, int zc) {
   const int V = quad_v(dtype, a.k), Q = (a.k + V - 1) / V, C = kQuadT / Q;
   const long long runs = (nxy + C - 1) / C;
   if (zc <= 0) {
-    // about kQuadBlocks workgroups (a plane more per march costs less than its two planes outside)
-    const long long chunks = (kQuadBlocks + runs - 1) / runs;
+    // the shortest marches whose workgroups are all resident at once
+    const long long per = (runs + 7) / 8 * 8, chunks = kQuadBlocks > per ? kQuadBlocks / per : 1;
     zc = (int)((a.nz + chunks - 1) / chunks);
   }
   if (zc > kQuadTab / C) zc = kQuadTab / C;

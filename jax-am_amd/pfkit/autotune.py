@@ -11,7 +11,8 @@ two, so nearby sizes share an entry.
 ``lookup`` consults, in order, the user cache ($PFKIT_AUTOTUNE_CACHE, default
 ``_autotune_cache.json`` next to this file; written by ``tune``) and the table shipped
 with the library (``tiles_mi355x.json``, produced on an MI355X by
-``python -m pfkit.autotune --sweep``), else returns the library defaults (-1, 0).
+``python -m pfkit.autotune --sweep``), else returns (-1, 0): the library chooses by size, K and
+dtype (pf_step).  The shipped table holds only shapes where a tuned entry is at least as fast as that.
 """
 import argparse
 import json
@@ -98,7 +99,8 @@ def candidates(pf_dtype, K, Nz):
     zcs = sorted({z for z in (0, 4, 8, 12, 16, 24, 32, Nz) if z <= Nz})
     # the same chunks with the lowest quarter of the planes in half-length chunks (dispatched last)
     zcs += [z | _lib.ZCHUNK_TAIL for z in (8, 12, 16, 24) if z < Nz]
-    return [(t, z) for t in range(max(nt, 1)) for z in zcs]
+    # the march of channel groups (tile -2), and every tile shape
+    return [(-2, z) for z in (0, 1, 2, 4, 8) if z <= Nz] + [(t, z) for t in range(max(nt, 1)) for z in zcs]
 
 
 def time_candidates(solver_rhs, eta, T, t_prev, dt, reps=20, warmup=3):

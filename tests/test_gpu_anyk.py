@@ -52,3 +52,26 @@ def test_rhs_reads_unaligned_states(cuda, dtype, k):
     buf = torch.rand(n * k + 1, device=cuda, generator=torch.Generator(cuda).manual_seed(k)).to(dtype)
     e = buf[1:].view(n, k)
     assert torch.equal(s.state_rhs(e, 0.1, [gaussian(nx, ny, nz)]), s.state_rhs(e.clone(), 0.1, [gaussian(nx, ny, nz)]))
+
+
+# both sides of the library's choice (channel groups / which tile) for tile -1, by dtype and K
+@pytest.mark.parametrize("dtype,k,dims", [
+    ("float32", 20, (64, 64, 22)), ("float32", 20, (64, 64, 24)), ("float32", 17, (57, 61, 30)), ("float32", 17, (57, 61, 31)),
+    ("float32", 10, (67, 63, 40)), ("float32", 2, (90, 70, 60)), ("bfloat16", 20, (64, 64, 24)), ("bfloat16", 10, (61, 50, 27)),
+    ("bfloat16", 12, (80, 60, 40)), ("float64", 10, (50, 50, 41)), ("float64", 10, (50, 50, 39)), ("float64", 16, (63, 50, 41)),
+    ("float64", 16, (63, 50, 45)), ("float64", 13, (91, 77, 85)), ("float64", 17, (33, 33, 20)), ("float64", 19, (91, 77, 62))])
+def test_library_choice_is_bitwise_the_tiled_step(cuda, dtype, k, dims):
+    nx, ny, nz = dims
+    a = args(nx, ny, nz, k, anisotropy=0.15, force_liquid=True)
+    pc = poly(nx, ny, nz, k, grains=20)
+    s = PFSolver(a, pc, dtype=dtype, device=cuda, clean=False, tile=-1, zchunk=0)
+    L = gaussian(nx, ny, nz)
+    eta = s.ini_cond()
+    eta[::3] += torch.rand(eta[::3].shape, device=cuda, generator=torch.Generator(cuda).manual_seed(k)).to(eta.dtype) * 0.2
+    outs = []
+    for tile, zc in ((-1, 0), (-1, 5), (-1, 0x10000), (0, 4), (-2, 0), (-2, 3)):
+        out = torch.empty_like(eta)
+        s.state_rhs.step(eta, out, L, 0.1, 0.101, tile, zc)
+        outs.append(out)
+    for o in outs[1:]:
+        assert torch.equal(o, outs[0])
