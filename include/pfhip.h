@@ -126,6 +126,18 @@ int pf_step(const void* eta_in_dev, void* eta_out_dev, int32_t dtype, const void
             int32_t tile, int32_t zchunk, void* stream);
 
 /*
+ * `steps` Euler steps in one call: no counterpart in the reference (a Python loop over stepper,
+ * applications/phase_field/simple/example.py:52-67).  Step i is pf_step from ts[i] to ts[i + 1] (ts: host
+ * array of steps + 1 times, read before the call returns) with the same temperature argument; the states
+ * go eta_in_dev -> buf0_dev -> buf1_dev -> buf0_dev ..., so the result is in buf0_dev for odd
+ * `steps` and in buf1_dev for even ones, and eta_in_dev is only read.  The three buffers must not
+ * alias.  Other arguments as pf_step.
+ */
+int pf_run(const void* eta_in_dev, void* buf0_dev, void* buf1_dev, int32_t dtype, const void* T_dev,
+           const pf_params_t* p, const void* axes_dev, const double* ts, int32_t steps, int32_t tile, int32_t zchunk,
+           void* stream);
+
+/*
  * Right-hand side only: rhs_out = state_rhs(eta_in, t, [T]) (allen_cahn.py:53-85), no Euler
  * update and no liquid reset.  Used by integrators other than explicit Euler (rk4,
  * allen_cahn.py:90-103).  Same arguments as pf_step; rhs_out has eta's dtype and shape.

@@ -344,6 +344,39 @@ static bool grid_ok(long long n, long long threads_per_item) {
   return (n + 255) / 256 * threads_per_item < (1LL << 31);
 }
 
+// The launch of a step: checks the arguments that do not concern the state buffers, fills the
+// instance description with the tiling and names the kernel.
+static int plan_step(const pf_params_t* p, int dtype, const void* T_dev, const void* axes_dev, int tile, int zchunk,
+                     StepDev& a, StepLaunch& fn) {
+  int rc = make_stepdev(p, dtype, T_dev, axes_dev, zchunk, a);
+  if (rc) return rc;
+  const bool aniso = p->anisotropy > 0.0;
+  if (tile < -2) return fail(PF_E_ARG, "tile must be >= -2");
+  const StepEntry* e = tile == -2 ? nullptr : find_entry(dtype, p->num_oris, aniso, tile);
+  const long long n = (long long)p->nz * p->ny * p->nx;
+  if (e) {
+    if (zchunk < 0 || (zchunk & ~(PF_ZCHUNK_TAIL | 0xffff)) != 0)
+      return fail(PF_E_ARG, "zchunk must be a plane count in [0, 65535], optionally | PF_ZCHUNK_TAIL");
+    if (march_fits(p, dtype)) return PF_E_ARG;
+    if (tile == -1) e = choose_step(dtype, p->num_oris, aniso, n);
+  } else if (tile > 0 && entry_count(dtype, p->num_oris, aniso) > 0) {
+    return fail(PF_E_ARG, "no such tile shape");
+  }
+  if (e) {
+    const long long cols = (long long)((p->nx + e->tx - 1) / e->tx) * ((p->ny + e->ty - 1) / e->ty);
+    if ((zchunk & 0xffff) == 0) zchunk |= fill_zchunk(p->nz, cols, held_workgroups(e));
+    set_tiles(a, e->tx, e->ty, zchunk);
+    const long long nt = (long long)a.tiles_x * a.tiles_y * a.tiles_z;
+    if (nt >= (1LL << 31)) return fail(PF_E_ARG, "too many tiles");
+    fn = e->step;
+  } else {
+    if (!grid_ok(n, 1)) return fail(PF_E_ARG, "grid too large for the generic kernel");
+    set_quads(a, dtype, zchunk > 0 ? zchunk & 0xffff : 0);
+    fn = generic_step(dtype, p->num_oris, aniso);
+  }
+  return PF_OK;
+}
+
 }  // namespace pf
 
 using namespace pf;
@@ -396,35 +429,33 @@ int pf_step(const void* eta_in_dev, void* eta_out_dev, int32_t dtype, const void
   if (((uintptr_t)eta_in_dev | (uintptr_t)eta_out_dev) & 15)
     return fail(PF_E_ARG, "eta buffers must be 16-byte aligned");
   StepDev a;
-  int rc = make_stepdev(p, dtype, T_dev, axes_dev, zchunk, a);
+  StepLaunch fn;
+  int rc = plan_step(p, dtype, T_dev, axes_dev, tile, zchunk, a, fn);
   if (rc) return rc;
-  const StepDyn d = make_dyn(a, eta_in_dev, eta_out_dev, t_prev, t_crt - t_prev);  // allen_cahn.py:112
-  const bool aniso = p->anisotropy > 0.0;
-  if (tile < -2) return fail(PF_E_ARG, "tile must be >= -2");
-  const StepEntry* e = tile == -2 ? nullptr : find_entry(dtype, p->num_oris, aniso, tile);
-  hipError_t err;
-  if (e) {
-    if (zchunk < 0 || (zchunk & ~(PF_ZCHUNK_TAIL | 0xffff)) != 0)
-      return fail(PF_E_ARG, "zchunk must be a plane count in [0, 65535], optionally | PF_ZCHUNK_TAIL");
-    if (march_fits(p, dtype)) return PF_E_ARG;
-    if (tile == -1) e = choose_step(dtype, p->num_oris, aniso, (long long)p->nz * p->ny * p->nx);
-  } else if (tile > 0 && entry_count(dtype, p->num_oris, aniso) > 0) {
-    return fail(PF_E_ARG, "no such tile shape");
+  hipError_t err = fn(a, make_dyn(a, eta_in_dev, eta_out_dev, t_prev, t_crt - t_prev), (hipStream_t)stream);  // allen_cahn.py:112
+  return err == hipSuccess ? PF_OK : hip_fail(err, "pf_step launch");
+}
+
+int pf_run(const void* eta_in_dev, void* buf0_dev, void* buf1_dev, int32_t dtype, const void* T_dev,
+           const pf_params_t* p, const void* axes_dev, const double* ts, int32_t steps, int32_t tile, int32_t zchunk,
+           void* stream) {
+  if (!eta_in_dev || !buf0_dev || !buf1_dev || !ts) return fail(PF_E_ARG, "NULL argument");
+  if (eta_in_dev == buf0_dev || eta_in_dev == buf1_dev || buf0_dev == buf1_dev)
+    return fail(PF_E_ARG, "eta_in and the two buffers must not alias");
+  if (((uintptr_t)eta_in_dev | (uintptr_t)buf0_dev | (uintptr_t)buf1_dev) & 15)
+    return fail(PF_E_ARG, "eta buffers must be 16-byte aligned");
+  if (steps < 1) return fail(PF_E_ARG, "steps must be >= 1");
+  StepDev a;
+  StepLaunch fn;
+  int rc = plan_step(p, dtype, T_dev, axes_dev, tile, zchunk, a, fn);
+  if (rc) return rc;
+  const void* in = eta_in_dev;
+  for (int i = 0; i < steps; ++i) {
+    void* out = i % 2 == 0 ? buf0_dev : buf1_dev;
+    hipError_t err = fn(a, make_dyn(a, in, out, ts[i], ts[i + 1] - ts[i]), (hipStream_t)stream);
+    if (err != hipSuccess) return hip_fail(err, "pf_run launch");
+    in = out;
   }
-  if (e) {
-    const long long cols = (long long)((p->nx + e->tx - 1) / e->tx) * ((p->ny + e->ty - 1) / e->ty);
-    if ((zchunk & 0xffff) == 0) zchunk |= fill_zchunk(p->nz, cols, held_workgroups(e));
-    set_tiles(a, e->tx, e->ty, zchunk);
-    const long long nt = (long long)a.tiles_x * a.tiles_y * a.tiles_z;
-    if (nt >= (1LL << 31)) return fail(PF_E_ARG, "too many tiles");
-    err = e->step(a, d, (hipStream_t)stream);
-  } else {
-    const long long n = (long long)p->nz * p->ny * p->nx;
-    if (!grid_ok(n, 1)) return fail(PF_E_ARG, "grid too large for the generic kernel");
-    set_quads(a, dtype, zchunk > 0 ? zchunk & 0xffff : 0);
-    err = generic_step(dtype, p->num_oris, aniso)(a, d, (hipStream_t)stream);
-  }
-  if (err != hipSuccess) return hip_fail(err, "pf_step launch");
   return PF_OK;
 }
 

@@ -70,6 +70,7 @@ SIGNATURES = {
     "pf_abi_sizes": (ctypes.c_int, [ctypes.POINTER(_SZ), ctypes.POINTER(_SZ), ctypes.POINTER(_SZ)]),
     "pf_device_count": (ctypes.c_int, []),
     "pf_step": (ctypes.c_int, [_VP, _VP, _I32, _VP, ctypes.POINTER(ParamsT), _VP, _D, _D, _I32, _I32, _VP]),
+    "pf_run": (ctypes.c_int, [_VP, _VP, _VP, _I32, _VP, ctypes.POINTER(ParamsT), _VP, _VP, _I32, _I32, _I32, _VP]),
     "pf_rhs": (ctypes.c_int, [_VP, _VP, _I32, _VP, ctypes.POINTER(ParamsT), _VP, _D, _VP]),
     "pf_tile_count": (ctypes.c_int, [_I32, _I32]),
     "pf_tile_shape": (ctypes.c_int, [_I32, _I32, _I32, ctypes.POINTER(_I32), ctypes.POINTER(_I32)]),

@@ -17,12 +17,18 @@ anisotropy         0.0      pf_params.yaml
 =================  =======  =========================================
 """
 import math
+from operator import itemgetter
 
 import yaml
 
 from . import _lib
 
 HARD_CODED = dict(gamma=1.0, T_clip=2000.0, zeta_sharpness=1e10, force_liquid=False, liquid_shift=1.0)
+
+
+# the values that make_params packs, as a tuple
+PACKED_KEYS = itemgetter("Nz", "Ny", "Nx", "num_oris", "m_g", "gamma", "kappa_g", "ad_hoc", "L0", "Qg", "gas_const",
+                         "T_liquidus", "T_clip", "zeta_sharpness", "anisotropy", "force_liquid", "liquid_shift")
 
 
 def yaml_parse(path):
