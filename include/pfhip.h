@@ -145,6 +145,15 @@ int pf_run(const void* eta_in_dev, void* buf0_dev, void* buf1_dev, int32_t dtype
 int pf_rhs(const void* eta_in_dev, void* rhs_out_dev, int32_t dtype, const void* T_dev,
            const pf_params_t* p, const void* axes_dev, double t, void* stream);
 
+/*
+ * One classical Runge-Kutta step (rk4, allen_cahn.py:90-103) from t_prev to t_crt, the temperature
+ * model evaluated at each stage's time; no liquid reset.  work_dev: [N, K] in `dtype`; sum_dev:
+ * [N, K] in the compute type (F64 when dtype == PF_F64, F32 otherwise).  Neither needs clearing; the
+ * four buffers must not alias.  PF_E_UNSUPPORTED for K > 512 (F32, BF16) or K > 256 (F64).
+ */
+int pf_rk4(const void* eta_in_dev, void* eta_out_dev, void* work_dev, void* sum_dev, int32_t dtype, const void* T_dev,
+           const pf_params_t* p, const void* axes_dev, double t_prev, double t_crt, void* stream);
+
 /* Tile shapes available for (dtype, K): count, (TX, TY) cells of shape `tile`, and the
  * threads per cell of shape `tile` (1, or 2 when a lane pair splits the K channels). */
 int pf_tile_count(int32_t dtype, int32_t k);

@@ -474,6 +474,32 @@ int pf_rhs(const void* eta_in_dev, void* rhs_out_dev, int32_t dtype, const void*
   return err == hipSuccess ? PF_OK : hip_fail(err, "pf_rhs launch");
 }
 
+int pf_rk4(const void* eta_in_dev, void* eta_out_dev, void* work_dev, void* sum_dev, int32_t dtype, const void* T_dev,
+           const pf_params_t* p, const void* axes_dev, double t_prev, double t_crt, void* stream) {
+  if (!eta_in_dev || !eta_out_dev || !work_dev || !sum_dev) return fail(PF_E_ARG, "NULL buffer");
+  const void* bufs[4] = {eta_in_dev, eta_out_dev, work_dev, sum_dev};
+  for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < i; ++j)
+      if (bufs[i] == bufs[j]) return fail(PF_E_ARG, "the buffers must not alias");
+  StepDev a;
+  int rc = make_stepdev(p, dtype, T_dev, axes_dev, 0, a);
+  if (rc) return rc;
+  if (!quad_fits(dtype, p->num_oris)) return fail(PF_E_UNSUPPORTED, "pf_rk4: too many orientations");
+  if (!grid_ok((long long)p->nz * p->ny * p->nx, 1)) return fail(PF_E_ARG, "grid too large");
+  set_quads(a, dtype, 0);
+  const double h = t_crt - t_prev;
+  const double t[4] = {t_prev, t_prev + h / 2.0, t_prev + h / 2.0, t_prev + h};  // allen_cahn.py:93-99
+  const double c[4] = {h / 2.0, h / 2.0, h, h / 6.0};
+  const void* in[4] = {eta_in_dev, work_dev, eta_out_dev, work_dev};
+  void* out[4] = {work_dev, eta_out_dev, work_dev, eta_out_dev};
+  for (int i = 0; i < 4; ++i) {
+    hipError_t err = rk_stage(a, make_dyn(a, in[i], out[i], t[i], 1.0), RkStage{eta_in_dev, sum_dev, c[i], i + 1}, dtype,
+                              p->anisotropy > 0.0, (hipStream_t)stream);
+    if (err != hipSuccess) return hip_fail(err, "pf_rk4 launch");
+  }
+  return PF_OK;
+}
+
 int pf_temperature(void* T_dev, int32_t T_dtype, const pf_params_t* p, double t, void* stream) {
   if (!T_dev) return fail(PF_E_ARG, "T buffer is NULL");
   if (T_dtype != PF_F64 && T_dtype != PF_F32) return fail(PF_E_ARG, "T dtype must be PF_F64 or PF_F32");

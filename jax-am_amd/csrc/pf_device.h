@@ -1266,12 +1266,24 @@ template <class TS, int V, bool TAIL> struct QuadAt {
 // instructions per channel: a wavefront's lanes hold different channels, so that a channel that is
 // zero everywhere can not be skipped as the tiled march does it (256x256x64, K = 20, FP32: 197 us
 // against 133 us there).
-// RHS = true writes state_rhs instead of the Euler update.
+// MODE: kStep the Euler update, kRhs state_rhs, kRk one stage of classical Runge-Kutta, whose
+// combinations of the stages' right-hand sides are formed where each is computed (RkStage).
+enum QuadMode { kStep, kRhs, kRk };
 constexpr int kQuadT = 256;
 constexpr int kQuadTab = 512;  // (cell, plane) pairs of a march at most
 
 template <class TC> struct QuadCoef {
   TC c1, A0, w1, w2;  // CellCoef without S (A = 4 gamma S + A0); isotropic: w1 = c2
+};
+
+// Stage i of a Runge-Kutta step from y0 with k_i = state_rhs(in): sum is k1 + 2 k2 + 2 k3 in the
+// compute type, written by stage 1 and updated by 2 and 3;
+//   stages 1 to 3: out = y0 + a k_i,   stage 4: out = y0 + a (sum + k_4).
+struct RkStage {
+  const void* y0;
+  void* sum;
+  double a;
+  int stage;
 };
 
 template <class TS, int V> struct QuadLds {
@@ -1292,8 +1304,8 @@ __device__ __forceinline__ bool quad_tile(const StepDev& a, int t, int& run, int
   return run < a.tiles_x;
 }
 
-template <class TS, bool ANISO, bool RHS, int V, bool TAIL>
-__device__ __forceinline__ void quad_march(const StepDev& a, const StepDyn& d, int run, int layer,
+template <class TS, bool ANISO, int MODE, int V, bool TAIL>
+__device__ __forceinline__ void quad_march(const StepDev& a, const StepDyn& d, const RkStage& rk, int run, int layer,
                                            QuadLds<TS, V>& lds, typename Traits<TS>::TC* __restrict__ ax) {
   using TC = typename Traits<TS>::TC;
   const int tid = threadIdx.x;
@@ -1341,14 +1353,26 @@ __device__ __forceinline__ void quad_march(const StepDev& a, const StepDyn& d, i
   inv_h2<TC>(a, ihx2, ihy2, ihz2);
   const TC g4 = (TC)a.gamma4;
   const int h = K / 2;
-  TS* o = (TS*)d.out + zb * plane + (long long)p * K;
+  using CV = VecA<TC, V, (int)sizeof(TC)>;
+  const long long at0 = zb * plane + (long long)p * K;
+  TS* o = (TS*)d.out + at0;
+  const TS* y0 = MODE == kRk ? (const TS*)rk.y0 + at0 : nullptr;
+  TC* sum = MODE == kRk ? (TC*)rk.sum + at0 : nullptr;
+  const TC ra = MODE == kRk ? (TC)rk.a : (TC)0;
   for (int l = 0; l < len; ++l) {
     const int z = zb + l;
     lo = c;
     c = n;
     TC* rows = lds.rows[l & 1];
-    QV xm, xp, ym, yp;
+    QV xm, xp, ym, yp, yc;
+    CV ks;
     if (on) {
+      if constexpr (MODE == kRk) {
+        if (rk.stage > 1) {
+          yc = at.raw(y0);
+          ks = *(const CV*)(sum + at.s);
+        }
+      }
       xm = at.raw(r + oxm);
       xp = at.raw(r + oxp);
       ym = at.raw(r + oym);
@@ -1376,32 +1400,55 @@ __device__ __forceinline__ void quad_march(const StepDev& a, const StepDyn& d, i
       cf.c2 = cf.w1 = q.w1;
       cf.w2 = q.w2;
       cf.A = fmac(g4, sum_sq_halves(s0, s1), q.A0);
-      cf.liquid = !RHS && lds.liquid[ci];
+      cf.liquid = MODE == kStep && lds.liquid[ci];
       const uint32_t key = sr_cell_key(sr_plane_key(d.seed, z), p) + (uint32_t)at.s * kSrChannel;
       QV res;
 #pragma unroll
       for (int e = 0; e < V; ++e) {
         const TC* axe = ax + 12 * (at.s + e);
-        const TC ce = to_tc(c.v[e]), x0 = to_tc(xm.v[e]), x1 = to_tc(xp.v[e]), y0 = to_tc(ym.v[e]),
-                 y1 = to_tc(yp.v[e]), z0 = to_tc(lo.v[e]), z1 = to_tc(n.v[e]);
+        const TC ce = to_tc(c.v[e]), x0 = to_tc(xm.v[e]), x1 = to_tc(xp.v[e]), w0 = to_tc(ym.v[e]),
+                 w1 = to_tc(yp.v[e]), z0 = to_tc(lo.v[e]), z1 = to_tc(n.v[e]);
         TC v;
-        if constexpr (RHS)
-          v = update_one<TC, ANISO, true>(cf, B, ihx2, ihy2, ihz2, ce, x0, x1, y0, y1, z0, z1, axe);
+        if constexpr (MODE != kStep)
+          v = update_one<TC, ANISO, true>(cf, B, ihx2, ihy2, ihz2, ce, x0, x1, w0, w1, z0, z1, axe);
         else
-          v = update_sr<TS, ANISO>(cf, B, ihx2, ihy2, ihz2, ce, x0, x1, y0, y1, z0, z1, axe,
+          v = update_sr<TS, ANISO>(cf, B, ihx2, ihy2, ihz2, ce, x0, x1, w0, w1, z0, z1, axe,
                                    key + (uint32_t)e * kSrChannel);
+        if constexpr (MODE == kRk) {
+          const TC k = v;
+          if (rk.stage == 1) {
+            ks.v[e] = k;
+            v = fmac(ra, k, ce);
+          } else if (rk.stage < 4) {
+            ks.v[e] = fmac((TC)2, k, ks.v[e]);
+            v = fmac(ra, k, to_tc(yc.v[e]));
+          } else {
+            v = fmac(ra, ks.v[e] + k, to_tc(yc.v[e]));
+          }
+        }
         res.v[e] = from_tc<TS>(cf.liquid ? (TC)0 : v);
       }
       if (!TAIL || at.e0 == 0) {
         *(QV*)(o + at.s) = res;
+        if constexpr (MODE == kRk)
+          if (rk.stage < 4) *(CV*)(sum + at.s) = ks;
       } else {
 #pragma unroll
-        for (int e = 1; e < V; ++e)
-          if (e >= at.e0) o[at.s + e] = res.v[e];
+        for (int e = 1; e < V; ++e) {
+          if (e >= at.e0) {
+            o[at.s + e] = res.v[e];
+            if constexpr (MODE == kRk)
+              if (rk.stage < 4) sum[at.s + e] = ks.v[e];
+          }
+        }
       }
     }
     r += plane;
     o += plane;
+    if constexpr (MODE == kRk) {
+      y0 += plane;
+      sum += plane;
+    }
   }
 }
 

@@ -155,6 +155,9 @@ const StepEntry* step_table_part_11(int* n);
 // of its threads' channel groups in one pass over the grid.
 long long set_quads(StepDev& a, int dtype, int zc);
 long long quad_threads(int dtype, int k, long long cells);
+bool quad_fits(int dtype, int k);  // K runs on the march of channel groups
+// one Runge-Kutta stage on the march of channel groups (quad_fits, set_quads)
+hipError_t rk_stage(const StepDev& a, const StepDyn& d, const RkStage& rk, int dtype, bool aniso, hipStream_t s);
 StepLaunch generic_step(int dtype, int k, bool aniso);
 StepLaunch generic_rhs(int dtype, int k, bool aniso);
 BatchLaunch generic_batch(int dtype, int k, bool aniso);

@@ -4,13 +4,13 @@
 
 namespace pf {
 
-template <class TS, bool ANISO, bool RHS, int V, bool TAIL>
-__global__ __launch_bounds__(kQuadT) void quad_kernel(const StepDev a, const StepDyn d) {
+template <class TS, bool ANISO, int MODE, int V, bool TAIL>
+__global__ __launch_bounds__(kQuadT) void quad_kernel(const StepDev a, const StepDyn d, const RkStage rk) {
   __shared__ QuadLds<TS, V> lds;
   extern __shared__ __attribute__((aligned(16))) char axmem[];
   int run, layer;
   if (quad_tile(a, blockIdx.x, run, layer))
-    quad_march<TS, ANISO, RHS, V, TAIL>(a, d, run, layer, lds, (typename Traits<TS>::TC*)axmem);
+    quad_march<TS, ANISO, MODE, V, TAIL>(a, d, rk, run, layer, lds, (typename Traits<TS>::TC*)axmem);
 }
 
 // Batched: work items are (slot, workgroup of the slot's own launch).
@@ -31,7 +31,8 @@ __global__ __launch_bounds__(kQuadT) void batch_quad_kernel(const StepDev* __res
     const StepDev& a = descs[it.slot];
     int run, layer;
     if (!quad_tile(a, it.tile, run, layer)) continue;
-    quad_march<TS, ANISO, false, V, TAIL>(a, dyns[it.slot], run, layer, lds, (typename Traits<TS>::TC*)axmem);
+    quad_march<TS, ANISO, kStep, V, TAIL>(a, dyns[it.slot], RkStage(), run, layer, lds,
+                                          (typename Traits<TS>::TC*)axmem);
     lds_barrier();  // LDS is reused by the next item
   }
 }
@@ -69,7 +70,7 @@ static int quad_v(int dtype, int K) {
   return K >= cap ? cap : 1;
 }
 // at most half a workgroup's threads per cell: the axis table of an anisotropic K stays under 25 KB
-static bool quad_fits(int dtype, int K) {
+bool quad_fits(int dtype, int K) {
   const int V = quad_v(dtype, K);
   return (K + V - 1) / V <= kQuadT / 2;
 }
@@ -102,17 +103,33 @@ long long set_quads(StepDev& a, int dtype, int zc) {
   return 8LL * a.tiles_y * a.tiles_z;
 }
 
-template <class TS, bool ANISO, bool RHS>
-static hipError_t launch_quad(const StepDev& a, const StepDyn& d, hipStream_t s) {
+template <class TS, bool ANISO, int MODE>
+static hipError_t launch_quad_mode(const StepDev& a, const StepDyn& d, const RkStage& rk, hipStream_t s) {
   using TC = typename Traits<TS>::TC;
   constexpr int dt = Traits<TS>::dtype;
   const unsigned nb = 8u * a.tiles_y * a.tiles_z;
   const size_t sh = ax_bytes(a.k, sizeof(TC), ANISO);
   const int V = quad_v(dt, a.k);
-  if (V == 1) quad_kernel<TS, ANISO, RHS, 1, false><<<nb, kQuadT, sh, s>>>(a, d);
-  else if (a.k % V == 0) quad_kernel<TS, ANISO, RHS, quad_cap<TS>(), false><<<nb, kQuadT, sh, s>>>(a, d);
-  else quad_kernel<TS, ANISO, RHS, quad_cap<TS>(), true><<<nb, kQuadT, sh, s>>>(a, d);
+  if (V == 1) quad_kernel<TS, ANISO, MODE, 1, false><<<nb, kQuadT, sh, s>>>(a, d, rk);
+  else if (a.k % V == 0) quad_kernel<TS, ANISO, MODE, quad_cap<TS>(), false><<<nb, kQuadT, sh, s>>>(a, d, rk);
+  else quad_kernel<TS, ANISO, MODE, quad_cap<TS>(), true><<<nb, kQuadT, sh, s>>>(a, d, rk);
   return hipGetLastError();
+}
+
+template <class TS, bool ANISO, bool RHS>
+static hipError_t launch_quad(const StepDev& a, const StepDyn& d, hipStream_t s) {
+  return launch_quad_mode<TS, ANISO, RHS ? kRhs : kStep>(a, d, RkStage(), s);
+}
+
+template <class TS>
+static hipError_t launch_rk(const StepDev& a, const StepDyn& d, const RkStage& rk, bool aniso, hipStream_t s) {
+  return aniso ? launch_quad_mode<TS, true, kRk>(a, d, rk, s) : launch_quad_mode<TS, false, kRk>(a, d, rk, s);
+}
+
+hipError_t rk_stage(const StepDev& a, const StepDyn& d, const RkStage& rk, int dtype, bool aniso, hipStream_t s) {
+  return dtype == PF_F64   ? launch_rk<double>(a, d, rk, aniso, s)
+         : dtype == PF_F32 ? launch_rk<float>(a, d, rk, aniso, s)
+                           : launch_rk<bf16_t>(a, d, rk, aniso, s);
 }
 
 template <class TS, bool ANISO, bool RHS>

@@ -72,6 +72,7 @@ SIGNATURES = {
     "pf_step": (ctypes.c_int, [_VP, _VP, _I32, _VP, ctypes.POINTER(ParamsT), _VP, _D, _D, _I32, _I32, _VP]),
     "pf_run": (ctypes.c_int, [_VP, _VP, _VP, _I32, _VP, ctypes.POINTER(ParamsT), _VP, _VP, _I32, _I32, _I32, _VP]),
     "pf_rhs": (ctypes.c_int, [_VP, _VP, _I32, _VP, ctypes.POINTER(ParamsT), _VP, _D, _VP]),
+    "pf_rk4": (ctypes.c_int, [_VP, _VP, _VP, _VP, _I32, _VP, ctypes.POINTER(ParamsT), _VP, _D, _D, _VP]),
     "pf_tile_count": (ctypes.c_int, [_I32, _I32]),
     "pf_tile_shape": (ctypes.c_int, [_I32, _I32, _I32, ctypes.POINTER(_I32), ctypes.POINTER(_I32)]),
     "pf_tile_lanes": (ctypes.c_int, [_I32, _I32, _I32]),

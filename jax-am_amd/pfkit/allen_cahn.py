@@ -114,6 +114,19 @@ class StateRHS:
                                _lib.ptr(self.axes), float(t_prev), float(t_crt), int(tile), int(zchunk),
                                _lib.stream_handle(self.device)), "pf_step")
 
+    def rk4_step(self, eta, T, t_prev, t_crt):
+        """One Runge-Kutta step (pf_rk4) into a new tensor; None when K is too large for it."""
+        p, Tptr = self.params_for(T)
+        out, work = torch.empty_like(eta), torch.empty_like(eta)
+        ksum = torch.empty(eta.shape, dtype=torch.float64 if self.dtype == torch.float64 else torch.float32,
+                           device=eta.device)
+        rc = _lib.load().pf_rk4(eta.data_ptr(), out.data_ptr(), work.data_ptr(), ksum.data_ptr(), self.pf_dtype, Tptr, p,
+                                _lib.ptr(self.axes), float(t_prev), float(t_crt), _lib.stream_handle(self.device))
+        if rc == _lib.PF_E_UNSUPPORTED:
+            return None
+        _lib.check(rc, "pf_rk4")
+        return out
+
 
 def phase_field(polycrystal, pf_args, dtype=None, device=None):
     """allen_cahn.py:10-87: returns the right-hand-side object for (polycrystal, pf_args)."""
@@ -131,9 +144,16 @@ def explicit_euler(state_pre, t_crt, f, ode_params):
 
 
 def rk4(state_pre, t_crt, f, ode_params):
-    """allen_cahn.py:90-103 (classical RK4 with four pf_rhs evaluations)."""
+    """allen_cahn.py:90-103 (classical RK4): four stage kernels that form the combinations of the
+    right-hand sides as they compute them (pf_rk4), or four pf_rhs evaluations where f is not a
+    plain StateRHS or has more orientations than those kernels take."""
     y_prev, t_prev = state_pre
     y_prev = f.check_state(y_prev)
+    if type(f) is StateRHS:
+        T, = ode_params
+        y = f.rk4_step(y_prev, T, t_prev, t_crt)
+        if y is not None:
+            return (y, t_crt), y
     h = t_crt - t_prev
     k1 = h * f(y_prev, t_prev, ode_params)
     k2 = h * f(y_prev + k1 / 2., t_prev + h / 2., ode_params)

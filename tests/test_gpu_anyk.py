@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import pf_oracle as O
-from pfkit import PFSolver
+from pfkit import PFSolver, rk4
 from problems import args, gaussian, poly, quench
 
 pytestmark = pytest.mark.gpu
@@ -75,3 +75,37 @@ def test_library_choice_is_bitwise_the_tiled_step(cuda, dtype, k, dims):
         outs.append(out)
     for o in outs[1:]:
         assert torch.equal(o, outs[0])
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nx,ny,nz,k", [(9, 7, 5, 1), (21, 10, 7, 5), (16, 16, 11, 16), (33, 5, 9, 17), (12, 11, 20, 20),
+                                        (4, 3, 3, 256), (3, 2, 2, 513)])
+def test_rk4_matches_the_oracle(cuda, dtype, nx, ny, nz, k):
+    a = args(nx, ny, nz, k, anisotropy=0.15)
+    pc = poly(nx, ny, nz, k)
+    n = nx * ny * nz
+    s = PFSolver(a, pc, dtype=dtype, device=cuda, clean=False)
+    rng = np.random.default_rng(k)
+    buf = torch.zeros(n * k + 1, dtype=dtype, device=cuda)
+    e = buf[1:].view(n, k)                      # aligned to one element only
+    e.copy_(torch.as_tensor(np.where(rng.random((n, k)) < 0.3, 0.0, rng.random((n, k)) / np.sqrt(k)), device=cuda))
+    ed = e.double().cpu().numpy()
+    T = rng.uniform(900.0, 1900.0, (n, 1))      # a temperature array is held over the step, as the oracle does
+    h = 2e-3
+    (got, t), _ = rk4((e, 0.1), 0.1 + h, s.state_rhs, [torch.as_tensor(T, device=cuda)])
+    want = O.rk4(ed, 0.1, 0.1 + h, T, a, pc.mesh_h_xyz, pc.unique_grain_directions)
+    assert t == 0.1 + h
+    # one rounding of the result to the storage type, stage states rounded alike times h |d rhs| << 1; FP64 as the step
+    tol = {torch.float64: 1e-12, torch.float32: 2e-6, torch.bfloat16: 2.0 ** -7}[dtype]
+    assert np.max(np.abs(got.double().cpu().numpy() - want)) <= tol * max(1.0, np.max(np.abs(want)))
+    # a source that moves within the step: the stages' own temperatures (four pf_rhs calls)
+    L = gaussian(nx, ny, nz)
+    f = lambda y, tt: s.state_rhs(y, tt, [L]).double()  # noqa: E731
+    y = e.double()
+    k1 = f(e, 0.1)
+    k2 = f((y + h / 2 * k1).to(dtype), 0.1 + h / 2)
+    k3 = f((y + h / 2 * k2).to(dtype), 0.1 + h / 2)
+    k4 = f((y + h * k3).to(dtype), 0.1 + h)
+    (got, _), _ = rk4((e, 0.1), 0.1 + h, s.state_rhs, [L])
+    ref = y + h / 6 * (k1 + 2 * k2 + 2 * k3 + k4)
+    assert float((got.double() - ref).abs().max()) <= tol * max(1.0, float(ref.abs().max()))
