@@ -288,8 +288,8 @@ int pf_batch_active(const pf_batch_t* b);
  * On return labels_dev[N] holds, per cell, the smallest cell index of its grain (-1 for liquid
  * cells); *n_grains grains exist; grain g (0 <= g < *n_grains, in no particular order) has root
  * cell root_dev[g] (capacity N) and cid_dev[root_dev[g]] == g (cid_dev: N entries).
- * ws_dev: 2 int32 of device scratch.  Label propagation passes run until one changes nothing
- * (at most max_passes, else PF_E_STATE).  Synchronizes the stream.
+ * ws_dev: 2 int32 of device scratch.  max_passes must be >= 1 (the labels are joined in one pass; it
+ * bounds nothing).  Synchronizes the stream.
  */
 int pf_segment(const int32_t* ori_dev, const void* T_dev, const pf_params_t* p, double t, int32_t* labels_dev,
                int32_t* cid_dev, int32_t* root_dev, int32_t* ws_dev, int64_t max_passes, int32_t* n_grains,

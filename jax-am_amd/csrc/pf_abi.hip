@@ -486,7 +486,7 @@ int pf_rk4(const void* eta_in_dev, void* eta_out_dev, void* work_dev, void* sum_
   if (rc) return rc;
   if (!quad_fits(dtype, p->num_oris)) return fail(PF_E_UNSUPPORTED, "pf_rk4: too many orientations");
   if (!grid_ok((long long)p->nz * p->ny * p->nx, 1)) return fail(PF_E_ARG, "grid too large");
-  set_quads(a, dtype, 0);
+  if (set_quads(a, dtype, 0) >= kQuadLaunch) return fail(PF_E_UNSUPPORTED, "pf_rk4: too many planes");
   const double h = t_crt - t_prev;
   const double t[4] = {t_prev, t_prev + h / 2.0, t_prev + h / 2.0, t_prev + h};  // allen_cahn.py:93-99
   const double c[4] = {h / 2.0, h / 2.0, h, h / 6.0};

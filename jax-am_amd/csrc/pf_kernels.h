@@ -154,6 +154,7 @@ const StepEntry* step_table_part_11(int* n);
 // number of workgroups (work items of the batched kernel) of a launch; quad_threads is the number
 // of its threads' channel groups in one pass over the grid.
 long long set_quads(StepDev& a, int dtype, int zc);
+constexpr long long kQuadLaunch = 1LL << 24;  // a launch has fewer workgroups of the march than this
 long long quad_threads(int dtype, int k, long long cells);
 bool quad_fits(int dtype, int k);  // K runs on the march of channel groups
 // one Runge-Kutta stage on the march of channel groups (quad_fits, set_quads)

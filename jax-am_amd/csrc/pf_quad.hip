@@ -103,6 +103,13 @@ long long set_quads(StepDev& a, int dtype, int zc) {
   return 8LL * a.tiles_y * a.tiles_z;
 }
 
+template <class TS, bool ANISO, bool RHS>
+static hipError_t launch_cells(const StepDev& a, const StepDyn& d, hipStream_t s) {
+  const long long n = (long long)a.nz * a.ny * a.nx;
+  generic_kernel<TS, ANISO, RHS><<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s>>>(a, d);
+  return hipGetLastError();
+}
+
 template <class TS, bool ANISO, int MODE>
 static hipError_t launch_quad_mode(const StepDev& a, const StepDyn& d, const RkStage& rk, hipStream_t s) {
   using TC = typename Traits<TS>::TC;
@@ -118,6 +125,8 @@ static hipError_t launch_quad_mode(const StepDev& a, const StepDyn& d, const RkS
 
 template <class TS, bool ANISO, bool RHS>
 static hipError_t launch_quad(const StepDev& a, const StepDyn& d, hipStream_t s) {
+  // a launch has fewer than 2^32 threads; planes of a few cells by very many planes would need more
+  if (8LL * a.tiles_y * a.tiles_z >= kQuadLaunch) return launch_cells<TS, ANISO, RHS>(a, d, s);
   return launch_quad_mode<TS, ANISO, RHS ? kRhs : kStep>(a, d, RkStage(), s);
 }
 
@@ -130,13 +139,6 @@ hipError_t rk_stage(const StepDev& a, const StepDyn& d, const RkStage& rk, int d
   return dtype == PF_F64   ? launch_rk<double>(a, d, rk, aniso, s)
          : dtype == PF_F32 ? launch_rk<float>(a, d, rk, aniso, s)
                            : launch_rk<bf16_t>(a, d, rk, aniso, s);
-}
-
-template <class TS, bool ANISO, bool RHS>
-static hipError_t launch_cells(const StepDev& a, const StepDyn& d, hipStream_t s) {
-  const long long n = (long long)a.nz * a.ny * a.nx;
-  generic_kernel<TS, ANISO, RHS><<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s>>>(a, d);
-  return hipGetLastError();
 }
 
 template <class TS, bool ANISO, int V, bool TAIL>

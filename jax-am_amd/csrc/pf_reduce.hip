@@ -431,7 +431,7 @@ int pf_argmax(const void* eta_dev, int32_t dtype, int64_t n_cells, int32_t k, in
   if ((n_cells + RB - 1) / RB >= (1LL << 31)) return fail(PF_E_ARG, "grid too large");
   hipStream_t s = (hipStream_t)stream;
   const int V = quad_of(dtype, k), Q = (k + V - 1) / V, C = Q <= RB ? RB / Q : 0;
-  if (C > 0 && (n_cells + C * AR - 1) / (C * AR) < (1LL << 31)) {
+  if (C > 0 && (n_cells + C * AR - 1) / (C * AR) < (1LL << 24)) {  // a launch has fewer than 2^32 threads
     switch (dtype) {
       case PF_F64: launch_argmax((const double*)eta_dev, n_cells, k, V, out_dev, s); break;
       case PF_F32: launch_argmax((const float*)eta_dev, n_cells, k, V, out_dev, s); break;

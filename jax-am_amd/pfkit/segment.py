@@ -5,7 +5,7 @@ The reference post-processes a written solution with ``process_eta``
 breadth-first search over face neighbours with the same orientation index (argmax eta)
 (:217-265); each grain gets its volume and an aspect ratio 2 l0 / (l1 + l2) from the PCA of its
 volume-weighted cell centroids (sklearn, explained variances l^2, descending; grains of fewer
-than 5 cells get 1) (:268-310).  Here the grains come from label propagation on the GPU
+than 5 cells get 1) (:268-310).  Here the grains come from joining labels on the GPU
 (libpfhip.so pf_segment) and the per-grain covariances from exact integer moments
 (pf_segment_moments); only the 3x3 eigenvalue problems run on the host.  Grains are listed in
 the reference's order: by orientation index, and within one orientation by their first cell.

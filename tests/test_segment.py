@@ -93,3 +93,60 @@ def test_gpu_segmentation_matches_oracle(shape, cuda):
         assert np.all(lab[g] == min(g))
     liquid = ~(T < a["T_liquidus"])
     assert np.all(lab[liquid] == -1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx,ny,nz,k", [(1, 1, 1, 1), (31, 7, 3, 2), (32, 8, 4, 2), (33, 9, 5, 2), (65, 17, 9, 3),
+                                        (100, 1, 1, 2), (1, 50, 33, 2), (64, 40, 37, 2)])
+@pytest.mark.parametrize("kind", ["noise", "one", "snake"])
+def test_labels_across_tiles(cuda, nx, ny, nz, k, kind):
+    """Labels, roots and moments where components wind through many tiles: random cells (hundreds of grains
+    to a tile, far more than its slots for moments), one component, and a comb whose teeth join at one
+    end.  Orientation values may be any int32.  Integer results: equal, not close."""
+    import ctypes
+    import torch
+    from scipy import ndimage
+    from pfkit import _lib
+    from pfkit.config import make_params
+    n = nx * ny * nz
+    rng = np.random.default_rng(n)
+    shape = (nz, ny, nx)
+    if kind == "noise":
+        ori = np.array([-7, 2 ** 31 - 1, -2 ** 31], np.int32)[rng.integers(0, k, shape)]
+    elif kind == "one":
+        ori = np.zeros(shape, np.int32)
+    else:
+        ori = (np.arange(ny)[None, :, None] % 2 + np.zeros(shape)).astype(np.int32)
+        ori[:, :, -1] = 0
+    T = rng.choice([300.0, 300.0, 300.0, 1700.0], n) if kind == "noise" else np.full(n, 300.0)
+    solid = T.reshape(shape) < 1623.0
+    want = np.full(shape, -1, np.int64)
+    idx = np.arange(n).reshape(shape)
+    for o in np.unique(ori):
+        lab, m = ndimage.label(solid & (ori == o))
+        if m:
+            first = ndimage.minimum(idx, lab, np.arange(1, m + 1)).astype(np.int64)
+            want[lab > 0] = first[lab[lab > 0] - 1]
+    a = args(nx, ny, nz, k)
+    p = make_params(a, (1.0, 1.0, 1.0), None)
+    p.laser.model, p.laser.T_dtype = _lib.PF_T_BUFFER, _lib.PF_F64
+    dev = lambda v: torch.as_tensor(v, device=cuda)  # noqa: E731
+    od, Td = dev(ori.reshape(-1)), dev(T)
+    out = [torch.full((n,), -9, dtype=torch.int32, device=cuda) for _ in range(3)]
+    ws, ng = torch.full((2,), 77, dtype=torch.int32, device=cuda), ctypes.c_int32(-1)
+    lib, st = _lib.load(), _lib.stream_handle(cuda)
+    _lib.check(lib.pf_segment(od.data_ptr(), Td.data_ptr(), p, 0.0, out[0].data_ptr(), out[1].data_ptr(),
+                              out[2].data_ptr(), ws.data_ptr(), 1, ctypes.byref(ng), st), "pf_segment")
+    labels, cid, root = (v.cpu().numpy() for v in out)
+    assert np.array_equal(labels, want.reshape(-1))
+    roots = np.unique(labels[labels >= 0])
+    assert ng.value == len(roots) and np.array_equal(np.sort(root[:ng.value]), roots)
+    assert np.array_equal(cid[root[:ng.value]], np.arange(ng.value))
+    if ng.value:
+        mom = torch.full((ng.value, 10), -5, dtype=torch.int64, device=cuda)
+        _lib.check(lib.pf_segment_moments(out[0].data_ptr(), out[1].data_ptr(), p, ng.value, mom.data_ptr(), st), "moments")
+        c = np.flatnonzero(labels >= 0)
+        z, y, x = np.unravel_index(c, shape)
+        cols = [np.ones_like(x), x, y, z, x * x, y * y, z * z, x * y, x * z, y * z]
+        ref = np.stack([np.bincount(cid[labels[c]], v, ng.value) for v in cols], axis=1).astype(np.int64)
+        assert np.array_equal(mom.cpu().numpy(), ref)
