@@ -254,7 +254,9 @@ typedef struct pf_batch_inst {
   const void* axes_dev;       /* [3, K, 3] like pf_step */
   int32_t dtype;
   int32_t tile;               /* tile shape index (-1 = default) */
-  int32_t zchunk;             /* 0 = default; optionally | PF_ZCHUNK_TAIL */
+  int32_t zchunk;             /* 0 = default; optionally | PF_ZCHUNK_TAIL.  Where an instance's class leaves
+                               * the GPU short of work the engine uses shorter marches, or the march of
+                               * channel groups (results do not depend on the tiling) */
   int32_t steps;              /* number of Euler steps to run */
   double t0, dt;              /* start time and fixed step */
   pf_params_t p;

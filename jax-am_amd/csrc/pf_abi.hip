@@ -124,7 +124,7 @@ int make_stepdev(const pf_params_t* p, int dtype, const void* T_dev, const void*
 namespace {
 struct Tables {
   std::vector<StepEntry> t[3];
-  std::unique_ptr<std::atomic<int>[]> held[3];  // per entry: workgroups the GPU holds at once (0: not asked yet)
+  std::unique_ptr<std::atomic<int>[]> held[3];  // per entry and kernel (step, batch): workgroups the GPU holds at once (0: not asked yet)
   Tables() {
     using PartFn = const StepEntry* (*)(int*);
     const PartFn parts[kInstParts] = {&step_table_part_0, &step_table_part_1, &step_table_part_2,
@@ -136,7 +136,7 @@ struct Tables {
       const StepEntry* e = f(&n);
       for (int i = 0; i < n; ++i) t[e[i].dtype].push_back(e[i]);
     }
-    for (int d = 0; d < 3; ++d) held[d] = std::make_unique<std::atomic<int>[]>(t[d].size());
+    for (int d = 0; d < 3; ++d) held[d] = std::make_unique<std::atomic<int>[]>(2 * t[d].size());
   }
 };
 const Tables& tables() {
@@ -163,14 +163,15 @@ const StepEntry* find_entry(int dtype, int k, bool aniso, int tile) {
   return nullptr;
 }
 
-// Workgroups of e's step kernel that the GPU holds at once (asked of the runtime once per kernel).
-static int held_workgroups(const StepEntry* e) {
+// Asked of the runtime once per kernel.
+int held_workgroups(const StepEntry* e, bool batch) {
   const Tables& tb = tables();
-  std::atomic<int>& c = tb.held[e->dtype][e - tb.t[e->dtype].data()];
+  std::atomic<int>& c = tb.held[e->dtype][2 * (e - tb.t[e->dtype].data()) + (batch ? 1 : 0)];
   int n = c.load(std::memory_order_relaxed);
   if (n == 0) {
     int per = 0, dev = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, e->kernel, e->tx * e->ty * e->h, 0) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, batch ? e->batch_kernel : e->kernel, e->tx * e->ty * e->h, 0) !=
+            hipSuccess ||
         hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
       (void)hipGetLastError();
@@ -206,14 +207,19 @@ static int fill_zchunk(int nz, long long cols, int held) {
 // 64x64x32 11.5/10.0; K = 17: 64x64x32 11.3/11.3, 64^3 17.5/14.2.  BF16 K = 20: 48x48x40 8.3/9.1; K = 10: 7.5/6.9;
 // K = 13: 64x64x32 9.1/9.3.  FP64 K = 10: 64x64x32 11.5/10.7 (isotropic 9.2/8.9), 48x48x40 9.3/10.2; K = 16: 64x64x32
 // 13.7/14.3, 64^3 20.3/21.2; K = 13: 96x96x48 30.9/33.2, 128x96x48 43.1/41.2; K = 17: 128x96x48 54.4/54.2.
-static const StepEntry* choose_step(int dtype, int k, bool aniso, long long cells) {
-  const long long t = quad_threads(dtype, k, cells);
+bool small_step(int dtype, int k, long long cells) {
+  if (!quad_fits(dtype, k)) return false;
   const bool odd = k % 2 != 0;
   long long most;
   if (dtype == PF_F64) most = odd && k >= 11 ? 4000000 : k >= 16 ? 1100000 : 500000;
   else if (dtype == PF_F32) most = odd ? 530000 : 470000;
   else most = odd || k >= 16 ? 480000 : 250000;
-  if (t <= most) return nullptr;
+  return quad_threads(dtype, k, cells) <= most;
+}
+
+static const StepEntry* choose_step(int dtype, int k, bool aniso, long long cells) {
+  if (small_step(dtype, k, cells)) return nullptr;
+  const bool odd = k % 2 != 0;
   int tile;
   if (dtype == PF_F64) tile = !odd ? 2 : k >= 17 ? 0 : 1;       // 16x4 lane pairs; 32x4; 16x4
   else if (k % 4 == 0 && k >= (dtype == PF_F32 ? 16 : 12)) tile = 4;  // 8x8 lane pairs (16-byte LDS reads need K % 4 = 0)
@@ -479,7 +485,7 @@ static int plan_step(const pf_params_t* p, int dtype, const void* T_dev, const v
   }
   if (e) {
     const long long cols = (long long)((p->nx + e->tx - 1) / e->tx) * ((p->ny + e->ty - 1) / e->ty);
-    if ((zchunk & 0xffff) == 0) zchunk |= fill_zchunk(p->nz, cols, held_workgroups(e));
+    if ((zchunk & 0xffff) == 0) zchunk |= fill_zchunk(p->nz, cols, held_workgroups(e, false));
     set_tiles(a, e->tx, e->ty, zchunk);
     const long long nt = (long long)a.tiles_x * a.tiles_y * a.tiles_z;
     if (nt >= (1LL << 31)) return fail(PF_E_ARG, "too many tiles");

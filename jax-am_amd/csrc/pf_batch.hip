@@ -1,15 +1,17 @@
 // Batched engine of libpfhip.so: many independent phase-field instances advanced
 // together.  Design:
 //   - Slot table (StepDev descriptors, BatchSlot step counters and each slot's StepDyn
-//     step arguments) lives in device memory; the device advances each slot's step
-//     index and ping-pong parity and rebuilds its StepDyn, so a captured graph stays
-//     valid while instances come and go.
+//     step arguments) lives in device memory; after each block of up to kPlan steps the device
+//     advances each slot's step index and ping-pong parity and plans its next kPlan steps,
+//     so a captured graph stays valid while instances come and go.
 //   - Instances are grouped into classes (dtype, K, anisotropy, tile shape).  Each
 //     class has a device-resident work list of (slot, tile) items walked by one
 //     persistent launch per step with a fixed grid.
-//   - `chunk` steps (launches of the classes that have work + advance) are captured
+//   - A class whose instances together leave the GPU short of workgroups runs shorter marches than its
+//     instances ask for, or the march of channel groups (rebuild_work).
+//   - `chunk` steps (launches of the classes that have work, an advance per block) are captured
 //     into one HIP graph and replayed.  Graphs are cached by (chunk, set of classes with
-//     work): admitting or removing an instance only rewrites table entries and work
+//     work and their kernels): admitting or removing an instance only rewrites table entries and work
 //     lists, and a new capture happens only for a class set not seen before.
 // Every tile of an instance runs exactly the per-cell arithmetic of pf_step with the
 // same tile shape, so an instance's trajectory does not depend on what else is in
@@ -24,40 +26,68 @@
 
 namespace pf {
 
-// After each step: advance every active slot's counters and build its next step's arguments;
-// a source-table slot also takes its next row's times and source into its description.
-__global__ __launch_bounds__(64) void advance_kernel(StepDev* __restrict__ descs, BatchSlot* __restrict__ slots,
-                                                    StepDyn* __restrict__ dyns, int n) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  BatchSlot b = slots[s];
-  if (b.active && b.steps_left > 0) {
-    const int done = b.n;
-    b.steps_left -= 1;
-    b.parity ^= 1;
-    b.n += 1;
-    if (b.path) {
-      b.tnow = b.path[PF_PATH_ROW * done + 1];
-      slots[s] = b;
-      if (b.steps_left > 0) {
-        StepDev a = descs[s];
-        const double* r = b.path + PF_PATH_ROW * b.n;
-        apply_path_row(a, r);
-        descs[s] = a;
-        dyns[s] = make_dyn(a, b.eta[b.parity], b.eta[b.parity ^ 1], r[0], r[1] - r[0]);
-      }
-    } else {
-      b.tnow = b.t0 + (double)b.n * b.dt;
-      slots[s] = b;
-      dyns[s] = slot_dyn(descs[s], b);
-    }
+// After a block of `steps` steps (0 when slots have come or gone): advance every active slot's counters
+// and plan its next kPlan steps.  A block's threads are eight slots by kPlan steps: every thread has read
+// its slot before the first of them writes it.  One launch per block of steps: one per step took
+// 5.0 us of each, for two dependent reads and a few stores.
+__global__ __launch_bounds__(8 * kPlan) void advance_kernel(StepDev* __restrict__ descs, BatchSlot* __restrict__ slots,
+                                                           StepDyn* __restrict__ dyns, int n, int steps) {
+  const int s = blockIdx.x * 8 + threadIdx.x / kPlan, i = threadIdx.x % kPlan;
+  BatchSlot b;
+  b.active = 0;
+  if (s < n) b = slots[s];
+  __syncthreads();
+  if (!b.active) return;
+  const int done = min(steps, b.steps_left);
+  if (done > 0) {
+    b.steps_left -= done;
+    b.parity ^= done & 1;
+    b.n += done;
+    b.tnow = b.path ? b.path[PF_PATH_ROW * (long long)(b.n - 1) + 1] : b.t0 + (double)b.n * b.dt;
+    if (i == 0) slots[s] = b;
   }
+  if (i >= b.steps_left) return;
+  const int m = b.n + i, par = b.parity ^ (i & 1);
+  StepDyn* d = dyns + i * n + s;
+  if (b.path) {
+    StepDev a = descs[s];
+    const double* r = b.path + PF_PATH_ROW * (long long)m;
+    apply_path_row(a, r);
+    descs[(1 + i) * n + s] = a;
+    *d = make_dyn(a, b.eta[par], b.eta[par ^ 1], r[0], r[1] - r[0]);
+  } else {
+    const double tp = b.t0 + (double)m * b.dt, tc = b.t0 + (double)(m + 1) * b.dt;
+    *d = make_dyn(descs[s], b.eta[par], b.eta[par ^ 1], tp, tc - tp);  // allen_cahn.py:112  h = t_crt - t_prev
+  }
+}
+
+// A slot's description and counters, passed by value: nothing of the caller's is read after the launch.
+__global__ void put_kernel(StepDev* desc, BatchSlot* slot, const StepDev a, const BatchSlot b) {
+  if (threadIdx.x == 0) *desc = a;
+  if (threadIdx.x == 1) *slot = b;
+}
+
+// Tiling of every slot (rebuild_work) into its description and those of its planned steps.
+struct SlotTiles {
+  int tiles_x, tiles_y, tiles_z, zc, zs, zsplit;
+};
+__global__ __launch_bounds__(64) void tiles_kernel(StepDev* __restrict__ descs, const SlotTiles* __restrict__ t, int n) {
+  const int s = blockIdx.x * 64 + threadIdx.x;
+  if (s >= n) return;
+  const SlotTiles v = t[s];
+  StepDev& a = descs[s];
+  a.tiles_x = v.tiles_x;
+  a.tiles_y = v.tiles_y;
+  a.tiles_z = v.tiles_z;
+  a.zc = v.zc;
+  a.zs = v.zs;
+  a.zsplit = v.zsplit;
 }
 
 struct BatchClass {
   int dtype, k, aniso, tile;
-  BatchLaunch fn;
-  int grid;
+  const StepEntry* entry;  // tile shape, null for K without tiled kernels
+  bool quads;              // the class runs the march of channel groups (always for a null entry)
   int off;    // offset of this class's work list in d_work
   int count;  // host copy of the work-item count
   int users;  // slots in this class; a class without users is retired and its index reused
@@ -66,8 +96,10 @@ struct BatchClass {
 struct SlotHost {
   bool used = false;
   int cls = -1;
-  int items = 0;   // work items of this slot
-  int charge = 0;  // what the slot counts for against max_tiles
+  int charge = 0;  // what the slot counts for against max_tiles: its tiles, or its blocks of 256 cells
+  int zchunk = 0;  // planes per march at most (0: the default), as the instance asked
+  int path = 0;    // 1: it has a source table
+  StepDev a;       // its description with the tiling it was given last
 };
 
 }  // namespace pf
@@ -84,12 +116,13 @@ struct pf_batch {
   WorkItem* d_work = nullptr;
   size_t work_cap = 0;     // items that d_work holds (at least max_tiles)
   int2* d_info = nullptr;  // per class (work-list offset, count)
+  SlotTiles* d_tiles = nullptr;
   std::vector<SlotHost> slots;
   std::vector<BatchClass> classes;
   bool work_dirty = false;
   struct Graph {
     int chunk;
-    unsigned long long mask;
+    unsigned long long mask, quads;  // classes with work, and those of them on channel groups
     hipGraph_t def;
     hipGraphExec_t exec;
   };
@@ -100,6 +133,8 @@ struct pf_batch {
 
 namespace {
 
+constexpr int kBatchQuads = 1024;  // workgroups of the batched march of channel groups on 256 CUs
+
 void drop_graphs(pf_batch* b) {
   for (pf_batch::Graph& g : b->graphs) {
     (void)hipGraphExecDestroy(g.exec);
@@ -108,13 +143,74 @@ void drop_graphs(pf_batch* b) {
   b->graphs.clear();
 }
 
+// Tiling of class c's slots.  A class with more than three fillings of the GPU (held workgroups) is tiled as its
+// instances asked (short marches balance the work, long ones read less: the autotuner's choice).  Below
+// that the length that ends with every CU busy is best: of the shortest marches that need one,
+// two and three fillings, the least fillings times planes (two more than a march writes are read).  A
+// class small enough for the march of channel groups (small_step) runs that.
+// Eight requests of 36x36x30 to 72x72x40 cells, K = 10, 16, 20, FP32: 80 us a step at the asked 6 and 8 planes,
+// 63 us here (of both without the scalar reads of constant_at; 52 us with them).
+void tile_class(pf_batch* b, int c) {
+  BatchClass& k = b->classes[c];
+  long long cells = 0;
+  for (const SlotHost& s : b->slots)
+    if (s.used && s.cls == c) cells += (long long)s.a.nz * s.a.ny * s.a.nx;
+  k.quads = !k.entry || small_step(k.dtype, k.k, cells);
+  if (k.quads) {
+    long long runs = 0;
+    for (SlotHost& s : b->slots)
+      if (s.used && s.cls == c) {
+        set_quads(s.a, k.dtype, 1);
+        runs += 8LL * s.a.tiles_y;
+      }
+    for (SlotHost& s : b->slots)
+      if (s.used && s.cls == c) {
+        const long long chunks = runs > 0 && kBatchQuads > runs ? kBatchQuads / runs : 1;
+        set_quads(s.a, k.dtype, (int)((s.a.nz + chunks - 1) / chunks));
+      }
+    return;
+  }
+  const int tx = k.entry->tx, ty = k.entry->ty;
+  const auto tile_all = [&](int zc) {  // 0: as asked
+    long long items = 0;
+    for (SlotHost& s : b->slots)
+      if (s.used && s.cls == c) {
+        set_tiles(s.a, tx, ty, zc == 0 || (s.zchunk & PF_ZCHUNK_TAIL) ? s.zchunk : zc);
+        items += (long long)s.a.tiles_x * s.a.tiles_y * s.a.tiles_z;
+      }
+    return items;
+  };
+  const long long held = held_workgroups(k.entry, true);
+  if (tile_all(0) > 3 * held) return;
+  int best = 0, best_cost = 0;
+  for (int m = 1, zc = 16; m <= 3; ++m) {
+    if (tile_all(zc) > m * held) continue;
+    while (zc > 2 && tile_all(zc - 1) <= m * held) --zc;
+    if (best == 0 || m * (zc + 2) < best_cost) {
+      best = zc;
+      best_cost = m * (zc + 2);
+    }
+  }
+  tile_all(best);
+}
+
 int rebuild_work(pf_batch* b) {
+  for (size_t c = 0; c < b->classes.size(); ++c)
+    if (b->classes[c].users > 0) tile_class(b, (int)c);
   // pack each class's work items contiguously, in slot order
   std::vector<std::vector<WorkItem>> per(b->classes.size());
+  std::vector<SlotTiles> tiles(b->max_inst, SlotTiles{0, 0, 0, 0, 0, 0});
   for (int s = 0; s < b->max_inst; ++s) {
     const SlotHost& sh = b->slots[s];
     if (!sh.used) continue;
-    for (int t = 0; t < sh.items; ++t) per[sh.cls].push_back(WorkItem{s, t});
+    const StepDev& a = sh.a;
+    tiles[s] = SlotTiles{a.tiles_x, a.tiles_y, a.tiles_z, a.zc, a.zs, a.zsplit};
+    const BatchClass& k = b->classes[sh.cls];
+    const long long items = !k.quads              ? (long long)a.tiles_x * a.tiles_y * a.tiles_z
+                            : quad_fits(k.dtype, k.k) ? 8LL * a.tiles_y * a.tiles_z
+                                                      : sh.charge;
+    if (items >= (1LL << 31)) return fail(PF_E_ARG, "instance too large");
+    for (int t = 0; t < (int)items; ++t) per[sh.cls].push_back(WorkItem{s, t, sh.path, 0});
   }
   std::vector<WorkItem> all;
   std::vector<int2> info(pf_batch::kMaxClasses, make_int2(0, 0));
@@ -126,8 +222,8 @@ int rebuild_work(pf_batch* b) {
   }
   hipError_t e = hipSuccess;
   if (all.size() > b->work_cap) {
-    // more items than max_tiles (slots are charged by the cells of a kernel of one thread per cell):
-    // a longer list; the graphs that hold the old one's address go with it
+    // more items than max_tiles, by which slots are charged as they asked to be tiled: a longer list;
+    // the graphs that hold the old one's address go with it
     WorkItem* grown = nullptr;
     const size_t cap = all.size() + all.size() / 2;
     e = hipMalloc((void**)&grown, sizeof(WorkItem) * cap);
@@ -143,6 +239,13 @@ int rebuild_work(pf_batch* b) {
     e = hipMemcpyAsync(b->d_work, all.data(), all.size() * sizeof(WorkItem), hipMemcpyHostToDevice, b->stream);
   if (e == hipSuccess)
     e = hipMemcpyAsync(b->d_info, info.data(), info.size() * sizeof(int2), hipMemcpyHostToDevice, b->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(b->d_tiles, tiles.data(), tiles.size() * sizeof(SlotTiles), hipMemcpyHostToDevice, b->stream);
+  if (e == hipSuccess) {
+    tiles_kernel<<<(b->max_inst + 63) / 64, 64, 0, b->stream>>>(b->d_desc, b->d_tiles, b->max_inst);
+    advance_kernel<<<(b->max_inst + 7) / 8, 8 * kPlan, 0, b->stream>>>(b->d_desc, b->d_slots, b->d_dyn, b->max_inst, 0);
+    e = hipGetLastError();
+  }
   // the host vectors above are pageable and local: finish the copies before they go away
   if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
   if (e != hipSuccess) return hip_fail(e, "pf_batch work-list upload");
@@ -157,16 +260,33 @@ unsigned long long active_mask(const pf_batch* b) {
   return m;
 }
 
-int launch_step_all(pf_batch* b) {
-  for (size_t c = 0; c < b->classes.size(); ++c) {
-    const BatchClass& k = b->classes[c];
-    if (k.count == 0) continue;
-    hipError_t e = k.fn(b->d_desc, b->d_dyn, b->d_slots, b->d_work, b->d_info, (int)c, k.grid, k.k, b->stream);
-    if (e != hipSuccess) return hip_fail(e, "pf_batch step launch");
+unsigned long long quad_mask(const pf_batch* b) {
+  unsigned long long m = 0;
+  for (size_t c = 0; c < b->classes.size(); ++c)
+    if (b->classes[c].count > 0 && b->classes[c].quads) m |= 1ULL << c;
+  return m;
+}
+
+// `steps` steps of every class with work, in blocks of up to kPlan with an advance after each.
+int launch_steps(pf_batch* b, int steps) {
+  const BatchView v{b->d_desc, b->d_dyn, b->d_slots, b->d_work, b->d_info, b->max_inst};
+  for (int done = 0; done < steps;) {
+    const int n = std::min(kPlan, steps - done);
+    for (int i = 0; i < n; ++i) {
+      for (size_t c = 0; c < b->classes.size(); ++c) {
+        const BatchClass& k = b->classes[c];
+        if (k.count == 0) continue;
+        const BatchLaunch fn = k.quads ? generic_batch(k.dtype, k.k, k.aniso != 0) : k.entry->batch;
+        hipError_t e = fn(v, (int)c, i, k.quads ? 2048 : 1024, k.k, b->stream);
+        if (e != hipSuccess) return hip_fail(e, "pf_batch step launch");
+      }
+    }
+    advance_kernel<<<(b->max_inst + 7) / 8, 8 * kPlan, 0, b->stream>>>(b->d_desc, b->d_slots, b->d_dyn, b->max_inst, n);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return hip_fail(e, "pf_batch advance launch");
+    done += n;
   }
-  advance_kernel<<<(b->max_inst + 63) / 64, 64, 0, b->stream>>>(b->d_desc, b->d_slots, b->d_dyn, b->max_inst);
-  hipError_t e = hipGetLastError();
-  return e == hipSuccess ? PF_OK : hip_fail(e, "pf_batch advance launch");
+  return PF_OK;
 }
 
 // Destroy the cached graphs that launch class c (its index is about to be retired).  The
@@ -186,9 +306,9 @@ void drop_graphs_of_class(pf_batch* b, int c) {
 
 // The graph of `chunk` steps for the current class set (captured on first use).
 int get_graph(pf_batch* b, int chunk, hipGraphExec_t* out) {
-  const unsigned long long mask = active_mask(b);
+  const unsigned long long mask = active_mask(b), quads = quad_mask(b);
   for (size_t i = 0; i < b->graphs.size(); ++i) {
-    if (b->graphs[i].chunk == chunk && b->graphs[i].mask == mask) {
+    if (b->graphs[i].chunk == chunk && b->graphs[i].mask == mask && b->graphs[i].quads == quads) {
       pf_batch::Graph g = b->graphs[i];
       b->graphs.erase(b->graphs.begin() + i);
       b->graphs.push_back(g);
@@ -198,8 +318,7 @@ int get_graph(pf_batch* b, int chunk, hipGraphExec_t* out) {
   }
   hipError_t e = hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) return hip_fail(e, "hipStreamBeginCapture");
-  int rc = PF_OK;
-  for (int i = 0; i < chunk && rc == PF_OK; ++i) rc = launch_step_all(b);
+  const int rc = launch_steps(b, chunk);
   hipGraph_t g = nullptr;
   e = hipStreamEndCapture(b->stream, &g);
   if (rc) {
@@ -220,7 +339,7 @@ int get_graph(pf_batch* b, int chunk, hipGraphExec_t* out) {
     (void)hipGraphDestroy(b->graphs.front().def);
     b->graphs.erase(b->graphs.begin());
   }
-  b->graphs.push_back(pf_batch::Graph{chunk, mask, g, ex});
+  b->graphs.push_back(pf_batch::Graph{chunk, mask, quads, g, ex});
   *out = ex;
   return PF_OK;
 }
@@ -240,11 +359,12 @@ pf_batch_t* pf_batch_create(int32_t max_instances, int32_t max_tiles, void* stre
   b->stream = (hipStream_t)stream;
   b->work_cap = max_tiles;
   b->slots.resize(max_instances);
-  hipError_t e = hipMalloc((void**)&b->d_desc, sizeof(StepDev) * max_instances);
-  if (e == hipSuccess) e = hipMalloc((void**)&b->d_dyn, sizeof(StepDyn) * max_instances);
+  hipError_t e = hipMalloc((void**)&b->d_desc, sizeof(StepDev) * (1 + kPlan) * max_instances);
+  if (e == hipSuccess) e = hipMalloc((void**)&b->d_dyn, sizeof(StepDyn) * kPlan * max_instances);
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_slots, sizeof(BatchSlot) * max_instances);
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_work, sizeof(WorkItem) * max_tiles);
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_info, sizeof(int2) * pf_batch::kMaxClasses);
+  if (e == hipSuccess) e = hipMalloc((void**)&b->d_tiles, sizeof(SlotTiles) * max_instances);
   if (e == hipSuccess) {
     std::vector<BatchSlot> z(max_instances);
     memset(z.data(), 0, z.size() * sizeof(BatchSlot));
@@ -271,6 +391,7 @@ void pf_batch_destroy(pf_batch_t* b) {
   if (b->d_slots) (void)hipFree(b->d_slots);
   if (b->d_work) (void)hipFree(b->d_work);
   if (b->d_info) (void)hipFree(b->d_info);
+  if (b->d_tiles) (void)hipFree(b->d_tiles);
   delete b;
 }
 
@@ -298,25 +419,18 @@ int pf_batch_add(pf_batch_t* b, const pf_batch_inst_t* inst) {
   if (rc) return rc;
   const bool aniso = inst->p.anisotropy > 0.0;
   const StepEntry* e = find_entry(inst->dtype, inst->p.num_oris, aniso, inst->tile);
-  int items, charge, tile = -1, grid;
-  BatchLaunch fn;
+  int charge, tile = -1;
   if (e) {
     if (march_fits(&inst->p, inst->dtype)) return PF_E_ARG;
     set_tiles(a, e->tx, e->ty, inst->zchunk);
-    items = charge = a.tiles_x * a.tiles_y * a.tiles_z;
+    charge = a.tiles_x * a.tiles_y * a.tiles_z;
     tile = e->tile;
-    fn = e->batch;
-    grid = 1024;
   } else {
     if (inst->tile > 0 && entry_count(inst->dtype, inst->p.num_oris, aniso) > 0)
       return fail(PF_E_ARG, "no such tile shape");
-    const long long n = set_quads(a, inst->dtype, 0);
-    if (n >= (1LL << 31) || ((long long)inst->p.nz * inst->p.ny * inst->p.nx + 255) / 256 >= (1LL << 31))
-      return fail(PF_E_ARG, "instance too large");
-    items = (int)n;
-    charge = (int)(((long long)inst->p.nz * inst->p.ny * inst->p.nx + 255) / 256);
-    fn = generic_batch(inst->dtype, inst->p.num_oris, aniso);
-    grid = 2048;
+    const long long n = (long long)inst->p.nz * inst->p.ny * inst->p.nx;
+    if ((n + 255) / 256 >= (1LL << 31)) return fail(PF_E_ARG, "instance too large");
+    charge = (int)((n + 255) / 256);
   }
   int total = 0;
   for (const SlotHost& sh : b->slots)
@@ -333,7 +447,7 @@ int pf_batch_add(pf_batch_t* b, const pf_batch_inst_t* inst) {
   }
   if (cls < 0) {
     // a new class takes a retired index (its graphs were dropped when it retired) or a new one
-    const BatchClass nc{inst->dtype, inst->p.num_oris, (int)aniso, tile, fn, grid, 0, 0, 0};
+    const BatchClass nc{inst->dtype, inst->p.num_oris, (int)aniso, tile, e, !e, 0, 0, 0};
     if (free_cls >= 0) {
       b->classes[free_cls] = nc;
       cls = free_cls;
@@ -356,26 +470,15 @@ int pf_batch_add(pf_batch_t* b, const pf_batch_inst_t* inst) {
   st.eta[1] = inst->eta_dev[1];
   st.tnow = inst->t0;
   st.path = inst->path_dev;
-  StepDyn dy = slot_dyn(a, st);
-  hipError_t he = hipSuccess;
-  if (inst->path_dev && inst->steps > 0) {  // the first row's times and source
-    double r0[PF_PATH_ROW];
-    he = hipMemcpyAsync(r0, inst->path_dev, sizeof(r0), hipMemcpyDeviceToHost, b->stream);
-    if (he == hipSuccess) he = hipStreamSynchronize(b->stream);
-    if (he != hipSuccess) return hip_fail(he, "pf_batch_add path");
-    apply_path_row(a, r0);
-    dy = make_dyn(a, st.eta[0], st.eta[1], r0[0], r0[1] - r0[0]);
-  }
-  he = hipMemcpyAsync(b->d_desc + slot, &a, sizeof(StepDev), hipMemcpyHostToDevice, b->stream);
-  if (he == hipSuccess) he = hipMemcpyAsync(b->d_dyn + slot, &dy, sizeof(StepDyn), hipMemcpyHostToDevice, b->stream);
-  if (he == hipSuccess)
-    he = hipMemcpyAsync(b->d_slots + slot, &st, sizeof(BatchSlot), hipMemcpyHostToDevice, b->stream);
-  if (he == hipSuccess) he = hipStreamSynchronize(b->stream);  // a, dy and st are locals
+  put_kernel<<<1, 64, 0, b->stream>>>(b->d_desc + slot, b->d_slots + slot, a, st);
+  hipError_t he = hipGetLastError();
   if (he != hipSuccess) return hip_fail(he, "pf_batch_add upload");
   b->slots[slot].used = true;
   b->slots[slot].cls = cls;
-  b->slots[slot].items = items;
   b->slots[slot].charge = charge;
+  b->slots[slot].zchunk = inst->zchunk;
+  b->slots[slot].path = inst->path_dev ? 1 : 0;
+  b->slots[slot].a = a;
   b->classes[cls].users += 1;
   b->work_dirty = true;
   return slot;
@@ -415,11 +518,7 @@ int pf_batch_run(pf_batch_t* b, int32_t steps, int32_t chunk) {
       if (e != hipSuccess) return hip_fail(e, "hipGraphLaunch");
     }
   }
-  for (; done < steps; ++done) {
-    int rc = launch_step_all(b);
-    if (rc) return rc;
-  }
-  return PF_OK;
+  return launch_steps(b, steps - done);
 }
 
 int pf_batch_status(pf_batch_t* b, int32_t* steps_left, double* t, int32_t* parity, int32_t n) {

@@ -26,6 +26,11 @@ int make_stepdev(const pf_params_t* p, int dtype, const void* T_dev, const void*
 // register-tiled instantiation; tile < 0 picks the default shape.
 const StepEntry* find_entry(int dtype, int k, bool aniso, int tile);
 int entry_count(int dtype, int k, bool aniso);
+// Workgroups of e's step (batch) kernel that the GPU holds at once.
+int held_workgroups(const StepEntry* e, bool batch);
+// Whether a step over `cells` cells of (dtype, k) (of all instances of a class together) is small enough for the
+// march of channel groups to beat the tiled kernels.
+bool small_step(int dtype, int k, long long cells);
 // default z-chunk for a grid and tile shape
 int default_zchunk(int nz, int ny, int nx, int tx, int ty);
 // fills the tile grid (tiles_x/y/z, zc) for a tile shape

@@ -44,13 +44,34 @@ __host__ __device__ inline void apply_path_row(StepDev& a, const double* r) {
 struct WorkItem {
   int slot;
   int tile;
+  int path;  // 1: the slot has a source table (its descriptions are planned per step)
+  int pad;
 };
 
-// Step arguments of slot s at its current step (allen_cahn.py:112  h = t_crt - t_prev).
-__host__ __device__ inline StepDyn slot_dyn(const StepDev& a, const BatchSlot& s) {
-  const double tp = s.t0 + (double)s.n * s.dt;
-  const double tc = s.t0 + (double)(s.n + 1) * s.dt;
-  return make_dyn(a, s.eta[s.parity], s.eta[s.parity ^ 1], tp, tc - tp);
+// The engine's device tables.  Slots change only between blocks of up to kPlan steps; the step arguments
+// of a block's steps, and the descriptions of slots with a source table (whose source differs from step
+// to step), are planned ahead by advance_kernel: dyns[i * inst + s] and descs[(1 + i) * inst + s] for
+// step i of the block, descs[s] for every other slot.
+constexpr int kPlan = 8;
+struct BatchView {
+  const StepDev* descs;
+  const StepDyn* dyns;
+  const BatchSlot* slots;
+  const WorkItem* work;
+  const int2* cinfo;  // per class (offset, count) of its work list
+  int inst;
+};
+
+// An element of a table in the constant address space.  A launch does not change the tables it reads,
+// but the compiler can not know: through ordinary pointers it reads what is uniform in a slot's description
+// again after the first barrier by per-lane loads, into vector registers.  Loads from this address
+// space are scalar and may be repeated anywhere, as those of kernel arguments.  A step of one 96x80x40,
+// K = 20, FP32 instance: 24.0 -> 20.7 us (16x8 tiles), 27.2 -> 21.4 us (8x8 lane pairs); 64 instances of 32^3 to
+// 128x128x64: 4.07e11 -> 4.27e11 updates/s with the engine's blocks of steps.
+template <class T>
+__device__ __forceinline__ const T& constant_at(const T* table, long long i) {
+  typedef const __attribute__((address_space(4))) T CT;
+  return *(const T*)((CT*)(uintptr_t)table + i);
 }
 
 template <int K, class TS, bool ANISO, int TX, int TY, int H>
@@ -69,42 +90,41 @@ __global__ __launch_bounds__(TX* TY* H) __attribute__((amdgpu_waves_per_eu(H + 1
 
 // Persistent batched step: a fixed grid walks the device-resident work list (slot,
 // tile) of one (dtype, K, anisotropy, tile shape) class.  Every workgroup exits after
-// the list is exhausted; slots with no steps left are skipped.  descs[slot] and
-// dyns[slot] are read in place (scalar loads), never copied into registers wholesale.
+// the list is exhausted; slots with no steps left are skipped.  Descriptions and step
+// arguments are read in place (scalar loads), never copied into registers wholesale.
 template <int K, class TS, bool ANISO, int TX, int TY, int H>
-__global__ __launch_bounds__(TX* TY* H) __attribute__((amdgpu_waves_per_eu(2))) void batch_kernel(
-    const StepDev* __restrict__ descs, const StepDyn* __restrict__ dyns, const BatchSlot* __restrict__ slots,
-    const WorkItem* __restrict__ work_all, const int2* __restrict__ cinfo, int cls) {
+__global__ __launch_bounds__(TX* TY* H) __attribute__((amdgpu_waves_per_eu(2))) void batch_kernel(const BatchView v, int cls, int step) {
   using TC = typename Traits<TS>::TC;
   using G = Tile<TS, K, TX, TY, H>;
   __shared__ __attribute__((aligned(16))) TC smem[G::NBUF * G::PSTR];
   __shared__ __attribute__((aligned(16))) TS stage[G::STAGE];
   __shared__ __attribute__((aligned(16))) TC ax[ANISO ? G::AXN : 4];
   __shared__ ZTab zt;
-  const int2 ci = cinfo[cls];  // (offset, count) of this class's work list
-  const WorkItem* __restrict__ work = work_all + ci.x;
+  const int2 ci = constant_at(v.cinfo, cls);  // (offset, count) of this class's work list
   for (int w = blockIdx.x; w < ci.y; w += gridDim.x) {
-    const WorkItem it = work[w];
-    const BatchSlot& s = slots[it.slot];
-    if (s.steps_left <= 0 || !s.active) continue;
-    const StepDev& a = descs[it.slot];
+    const WorkItem it = constant_at(v.work, ci.x + w);
+    const BatchSlot& s = constant_at(v.slots, it.slot);
+    const StepDev& a = constant_at(v.descs, it.path ? (1LL + step) * v.inst + it.slot : it.slot);
+    const StepDyn& d = constant_at(v.dyns, (long long)step * v.inst + it.slot);
+    if (s.steps_left <= step || !s.active) continue;
     int tx, ty, tz;
     tile_coords(it.tile, a.tiles_x, a.tiles_y, a.tiles_z, tx, ty, tz);
-    march_tile<K, TS, ANISO, TX, TY, H>(a, dyns[it.slot], tx, ty, tz, smem, stage, ax, &zt);
+    march_tile<K, TS, ANISO, TX, TY, H>(a, d, tx, ty, tz, smem, stage, ax, &zt);
     lds_barrier();  // LDS is reused by the next tile
   }
 }
 
 using StepLaunch = hipError_t (*)(const StepDev&, const StepDyn&, hipStream_t);
-using BatchLaunch = hipError_t (*)(const StepDev*, const StepDyn*, const BatchSlot*, const WorkItem*, const int2*,
-                                   int cls, int grid, int k, hipStream_t);
+// Step `i` of the block for class `cls` (k: its number of orientations).
+using BatchLaunch = hipError_t (*)(const BatchView&, int cls, int i, int grid, int k, hipStream_t);
 
 struct StepEntry {
   int dtype, k, aniso, tile, tx, ty, h;
   StepLaunch step;
   BatchLaunch batch;
   size_t lds;
-  const void* kernel;  // the step kernel (occupancy queries)
+  const void* kernel;        // the step and batch kernels (occupancy queries)
+  const void* batch_kernel;
 };
 
 template <int K, class TS, bool ANISO, int TX, int TY, int H>
@@ -115,9 +135,8 @@ hipError_t launch_step(const StepDev& a, const StepDyn& d, hipStream_t s) {
 }
 
 template <int K, class TS, bool ANISO, int TX, int TY, int H>
-hipError_t launch_batch(const StepDev* a, const StepDyn* d, const BatchSlot* sl, const WorkItem* w, const int2* ci,
-                        int cls, int grid, int, hipStream_t s) {
-  batch_kernel<K, TS, ANISO, TX, TY, H><<<dim3(grid), dim3(TX * TY * H), 0, s>>>(a, d, sl, w, ci, cls);
+hipError_t launch_batch(const BatchView& v, int cls, int i, int grid, int, hipStream_t s) {
+  batch_kernel<K, TS, ANISO, TX, TY, H><<<dim3(grid), dim3(TX * TY * H), 0, s>>>(v, cls, i);
   return hipGetLastError();
 }
 
@@ -132,7 +151,8 @@ hipError_t launch_batch(const StepDev* a, const StepDyn* d, const BatchSlot* sl,
    &launch_step<K, TS, (A != 0), TX, TY, H>,                                     \
    &launch_batch<K, TS, (A != 0), TX, TY, H>,                                    \
    Tile<TS, K, TX, TY, H>::LDS_BYTES,                                            \
-   (const void*)&step_kernel<K, TS, (A != 0), TX, TY, H>}
+   (const void*)&step_kernel<K, TS, (A != 0), TX, TY, H>,                         \
+   (const void*)&batch_kernel<K, TS, (A != 0), TX, TY, H>}
 
 // instantiation tables, one per compiled part of pf_inst.hip (see Makefile):
 // parts 0-3 F32, 4-7 BF16, 8-11 F64, each over a K range
@@ -154,6 +174,7 @@ const StepEntry* step_table_part_11(int* n);
 // number of workgroups (work items of the batched kernel) of a launch; quad_threads is the number
 // of its threads' channel groups in one pass over the grid.
 long long set_quads(StepDev& a, int dtype, int zc);
+constexpr int kQuadBlocks = 1280;  // five workgroups of the march on each of 256 CUs (what the registers allow)
 constexpr long long kQuadLaunch = 1LL << 24;  // a launch has fewer workgroups of the march than this
 long long quad_threads(int dtype, int k, long long cells);
 bool quad_fits(int dtype, int k);  // K runs on the march of channel groups

@@ -15,24 +15,20 @@ __global__ __launch_bounds__(kQuadT) void quad_kernel(const StepDev a, const Ste
 
 // Batched: work items are (slot, workgroup of the slot's own launch).
 template <class TS, bool ANISO, int V, bool TAIL>
-__global__ __launch_bounds__(kQuadT) void batch_quad_kernel(const StepDev* __restrict__ descs,
-                                                           const StepDyn* __restrict__ dyns,
-                                                           const BatchSlot* __restrict__ slots,
-                                                           const WorkItem* __restrict__ work_all,
-                                                           const int2* __restrict__ cinfo, int cls) {
+__global__ __launch_bounds__(kQuadT) void batch_quad_kernel(const BatchView v, int cls, int step) {
   __shared__ QuadLds<TS, V> lds;
   extern __shared__ __attribute__((aligned(16))) char axmem[];
-  const int2 ci = cinfo[cls];
-  const WorkItem* __restrict__ work = work_all + ci.x;
+  const int2 ci = constant_at(v.cinfo, cls);
   for (int w = blockIdx.x; w < ci.y; w += gridDim.x) {
-    const WorkItem it = work[w];
-    const BatchSlot& s = slots[it.slot];
-    if (s.steps_left <= 0 || !s.active) continue;
-    const StepDev& a = descs[it.slot];
+    const WorkItem it = constant_at(v.work, ci.x + w);
+    const BatchSlot& s = constant_at(v.slots, it.slot);
+    const StepDev& a = constant_at(v.descs, it.path ? (1LL + step) * v.inst + it.slot : it.slot);
+    const StepDyn& d = constant_at(v.dyns, (long long)step * v.inst + it.slot);
+    if (s.steps_left <= step || !s.active) continue;
     int run, layer;
     if (!quad_tile(a, it.tile, run, layer)) continue;
-    quad_march<TS, ANISO, kStep, V, TAIL>(a, dyns[it.slot], RkStage(), run, layer, lds,
-                                          (typename Traits<TS>::TC*)axmem);
+    quad_march<TS, ANISO, kStep, V, TAIL>(a, d, RkStage(), run, layer, lds,
+                                              (typename Traits<TS>::TC*)axmem);
     lds_barrier();  // LDS is reused by the next item
   }
 }
@@ -46,21 +42,17 @@ __global__ __launch_bounds__(256) void generic_kernel(const StepDev a, const Ste
 
 // Batched, one thread per cell: work items are (slot, block of 256 cells).
 template <class TS, bool ANISO>
-__global__ __launch_bounds__(256) void batch_generic_kernel(const StepDev* __restrict__ descs,
-                                                           const StepDyn* __restrict__ dyns,
-                                                           const BatchSlot* __restrict__ slots,
-                                                           const WorkItem* __restrict__ work_all,
-                                                           const int2* __restrict__ cinfo, int cls) {
-  const int2 ci = cinfo[cls];
-  const WorkItem* __restrict__ work = work_all + ci.x;
+__global__ __launch_bounds__(256) void batch_generic_kernel(const BatchView v, int cls, int step) {
+  const int2 ci = constant_at(v.cinfo, cls);
   for (int w = blockIdx.x; w < ci.y; w += gridDim.x) {
-    const WorkItem it = work[w];
-    const BatchSlot& s = slots[it.slot];
-    if (s.steps_left <= 0 || !s.active) continue;
-    const StepDev& a = descs[it.slot];
+    const WorkItem it = constant_at(v.work, ci.x + w);
+    const BatchSlot& s = constant_at(v.slots, it.slot);
+    const StepDev& a = constant_at(v.descs, it.path ? (1LL + step) * v.inst + it.slot : it.slot);
+    const StepDyn& d = constant_at(v.dyns, (long long)step * v.inst + it.slot);
+    if (s.steps_left <= step || !s.active) continue;
     const long long n = (long long)a.nz * a.ny * a.nx;
     const long long cell = (long long)it.tile * 256 + threadIdx.x;
-    if (cell < n) generic_cell<TS, ANISO>(a, dyns[it.slot], cell);
+    if (cell < n) generic_cell<TS, ANISO>(a, d, cell);
   }
 }
 
@@ -74,8 +66,6 @@ bool quad_fits(int dtype, int K) {
   const int V = quad_v(dtype, K);
   return (K + V - 1) / V <= kQuadT / 2;
 }
-constexpr int kQuadBlocks = 1280;  // five workgroups on each of 256 CUs (what the registers allow)
-
 static size_t ax_bytes(int k, int tc, bool aniso) { return aniso ? (size_t)12 * k * tc : 16; }
 
 long long quad_threads(int dtype, int k, long long cells) {
@@ -142,17 +132,15 @@ hipError_t rk_stage(const StepDev& a, const StepDyn& d, const RkStage& rk, int d
 }
 
 template <class TS, bool ANISO, int V, bool TAIL>
-static hipError_t launch_batch_quad(const StepDev* a, const StepDyn* d, const BatchSlot* sl, const WorkItem* w,
-                                    const int2* ci, int cls, int grid, int k, hipStream_t s) {
+static hipError_t launch_batch_quad(const BatchView& v, int cls, int i, int grid, int k, hipStream_t s) {
   batch_quad_kernel<TS, ANISO, V, TAIL>
-      <<<dim3(grid), dim3(kQuadT), ax_bytes(k, sizeof(typename Traits<TS>::TC), ANISO), s>>>(a, d, sl, w, ci, cls);
+      <<<dim3(grid), dim3(kQuadT), ax_bytes(k, sizeof(typename Traits<TS>::TC), ANISO), s>>>(v, cls, i);
   return hipGetLastError();
 }
 
 template <class TS, bool ANISO>
-static hipError_t launch_batch_cells(const StepDev* a, const StepDyn* d, const BatchSlot* sl, const WorkItem* w,
-                                     const int2* ci, int cls, int grid, int, hipStream_t s) {
-  batch_generic_kernel<TS, ANISO><<<dim3(grid), dim3(256), 0, s>>>(a, d, sl, w, ci, cls);
+static hipError_t launch_batch_cells(const BatchView& v, int cls, int i, int grid, int, hipStream_t s) {
+  batch_generic_kernel<TS, ANISO><<<dim3(grid), dim3(256), 0, s>>>(v, cls, i);
   return hipGetLastError();
 }
 

@@ -1,0 +1,97 @@
+"""GPU tests of the batch engine's blocks of planned steps and of the kernels it chooses per class: every instance's state
+bitwise the same as its own run, whatever shares its launches."""
+import pytest
+import torch
+
+from pfkit import PFSolver, workloads
+from pfkit.batch import BatchEngine
+from pfkit.laser import RosenthalRamp
+
+pytestmark = pytest.mark.gpu
+
+
+def _solo(w, steps):
+    s = PFSolver(w.pf_args, w.polycrystal, dtype=w.dtype, clean=False, tile=-2, zchunk=0)
+    return s.run(s.ini_cond(), w.ts(steps), w.laser)
+
+
+def _make(j, nx, ny, nz, k, dtype, steps, aniso=0.15):
+    return workloads.make(f"b{j}", nx, ny, nz, k, 10, steps, dtype, aniso, seed=80 + j, vel=2.0)
+
+
+@pytest.mark.parametrize("chunk", [0, 1, 5, 8, 11, 16, 20])
+def test_step_counts_within_and_across_blocks(cuda, chunk):
+    steps = (0, 1, 7, 8, 9, 17, 24)
+    W = [_make(j, 18 + j, 11, 9, 6, "float32", n) for j, n in enumerate(steps)]
+    eng = BatchEngine(max_instances=8)
+    slots = [eng.add(w.instance()) for w in W]
+    eng.run(25, chunk)
+    left, t, parity = eng.status()
+    for w, s, n in zip(W, slots, steps):
+        assert left[s] == 0 and t[s] == n * w.dt
+        assert torch.equal(eng.state(s, parity[s]), _solo(w, n))
+    eng.close()
+
+
+@pytest.mark.parametrize("dtype,k", [("float32", 10), ("bfloat16", 12), ("float64", 13), ("float32", 27)])
+def test_a_class_changes_its_kernel_as_instances_come_and_go(cuda, dtype, k):
+    """One small instance runs on channel groups; with large ones in its class on tiles of one, two or three
+    fillings and then as asked; alone again, on channel groups: graphs of each are cached."""
+    small = _make(0, 24, 20, 13, k, dtype, 40)
+    big = [_make(1 + j, 130, 128, 40, k, dtype, 8) for j in range(4)]
+    eng = BatchEngine(max_instances=8)
+    s0 = eng.add(small.instance())
+    done = 0
+    for n in (0, 1, 2, 4, 0, 1):
+        slots = [eng.add(w.instance()) for w in big[:n]]
+        eng.run(6, 6)
+        done += 6
+        par = eng.status()[2]
+        assert torch.equal(eng.state(s0, par[s0]), _solo(small, done))
+        for w, s in zip(big, slots):
+            assert torch.equal(eng.state(s, par[s]), _solo(w, 6))
+            eng.remove(s)
+    eng.close()
+
+
+def test_more_work_items_than_max_tiles(cuda):
+    """Slots are charged as they asked to be tiled; shorter marches and channel groups make more work items than that,
+    and the work list grows (between replays of graphs that held the shorter one)."""
+    W = [_make(j, 33, 31, 24, 25, "float32", 20) for j in range(3)]
+    charge = (33 * 31 * 24 + 255) // 256
+    eng = BatchEngine(max_instances=4, max_tiles=3 * charge)
+    slots = [eng.add(W[0].instance())]
+    eng.run(4, 4)
+    slots += [eng.add(w.instance()) for w in W[1:]]
+    eng.run(4, 4)
+    par = eng.status()[2]
+    for w, s, n in zip(W, slots, (8, 4, 4)):
+        assert torch.equal(eng.state(s, par[s]), _solo(w, n))
+    eng.close()
+
+
+@pytest.mark.parametrize("chunk", [3, 16])
+def test_source_tables_are_planned_per_step(cuda, chunk):
+    """Two instances of one class with source tables of their own and one without, over steps that end within a
+    block: each bitwise its own run_toolpath or run."""
+    W = [_make(j, 26, 18, 10, 8, "float32", 19) for j in range(3)]
+    n, dt = 19, W[0].dt
+    ramps = [RosenthalRamp(x0=5.0, y0=9.0, z0=10.0, t_OFF=30 * dt * (1 + 0.1 * j), dt=dt * (1 + 0.1 * j),
+                           vel_avg=0.3 / dt, Q_max=2.0e6, Q_min=0.5e6, alpha=5.2) for j in range(2)]
+    eng = BatchEngine(max_instances=4)
+    slots = []
+    for w, r in zip(W, ramps):
+        inst = w.instance(toolpath=r)
+        slots.append(eng.add(inst))
+    slots.append(eng.add(W[2].instance()))
+    eng.run(n, chunk)
+    left, t, par = eng.status()
+    for j, (w, s) in enumerate(zip(W, slots)):
+        if j < 2:
+            sol = PFSolver(w.pf_args, w.polycrystal, dtype="float32", clean=False)
+            want = sol.run_toolpath(sol.ini_cond(), ramps[j], steps=n)
+            assert t[s] == ramps[j].step_times()[n]
+        else:
+            want = _solo(w, n)
+        assert left[s] == 0 and torch.equal(eng.state(s, par[s]), want)
+    eng.close()
