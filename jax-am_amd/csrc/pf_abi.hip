@@ -188,9 +188,12 @@ int held_workgroups(const StepEntry* e, bool batch) {
 // that fill it a whole number of times, once if they then have at most 12 planes, else as often as
 // that takes.  Each march reads two planes more than it writes, so longer is better, but only while
 // no CU idles at the launch's end: 128x96x48, K = 20, FP64 (16x4 lane pairs) 46.6 us at 12 planes, one
-// filling, against 51.4 at 6; 203x197x59, K = 17, FP32 (16x8) 87.7 us at 10, two fillings, against 91.4 at 8
-// and 100.3 at 16.
+// filling, against 51.4 at 6; 203x197x59, K = 17, FP32 (16x8) 85.8 us at 10, two fillings, against 98 at 16.
+// A tall grid whose columns alone fill the GPU's half takes 16 planes with the tail split (PF_ZCHUNK_TAIL), whose
+// short marches end the launch: 256x256x64 in FP32 K = 13 104.6 -> 100.0 us, BF16 K = 10 57.8 -> 54.4, K = 17 112.2 -> 105.7, FP64
+// K = 12 189 -> 182.5, against fillings; on 203x197x59 (a third) it is slower, FP32 K = 17 91 against 85.8.
 static int fill_zchunk(int nz, long long cols, int held) {
+  if (nz >= 40 && 2 * cols >= held) return 16 | PF_ZCHUNK_TAIL;
   const long long kmin = (nz + 11) / 12;
   const long long m = (kmin * cols + held - 1) / held;  // fillings: the fewest whose chunks have at most 12 planes
   const long long k = m * held / cols;
@@ -222,8 +225,10 @@ static const StepEntry* choose_step(int dtype, int k, bool aniso, long long cell
   const bool odd = k % 2 != 0;
   int tile;
   if (dtype == PF_F64) tile = !odd ? 2 : k >= 17 ? 0 : 1;       // 16x4 lane pairs; 32x4; 16x4
-  else if (k % 4 == 0 && k >= (dtype == PF_F32 ? 16 : 12)) tile = 4;  // 8x8 lane pairs (16-byte LDS reads need K % 4 = 0)
-  else tile = 2;                                                // 16x8
+  else if (k % 4 == 0 && (k >= 16 || (dtype == PF_BF16 && k == 12 && cells < 2000000)))
+    tile = 4;  // 8x8 lane pairs (whole vectors in each half need K % 4 = 0; BF16 K = 12: 256x256x64 65.1 against 58.9 us)
+  else
+    tile = 2;  // 16x8
   const StepEntry* e = find_entry(dtype, k, aniso, tile);
   return e ? e : find_entry(dtype, k, aniso, 0);
 }
@@ -487,8 +492,7 @@ static int plan_step(const pf_params_t* p, int dtype, const void* T_dev, const v
     const long long cols = (long long)((p->nx + e->tx - 1) / e->tx) * ((p->ny + e->ty - 1) / e->ty);
     if ((zchunk & 0xffff) == 0) zchunk |= fill_zchunk(p->nz, cols, held_workgroups(e, false));
     set_tiles(a, e->tx, e->ty, zchunk);
-    const long long nt = (long long)a.tiles_x * a.tiles_y * a.tiles_z;
-    if (nt >= (1LL << 31)) return fail(PF_E_ARG, "too many tiles");
+    if (tile_launch(a.tiles_x, a.tiles_y, a.tiles_z) >= (1LL << 31)) return fail(PF_E_ARG, "too many tiles");
     fn = e->step;
   } else {
     if (!grid_ok(n, 1)) return fail(PF_E_ARG, "grid too large for the generic kernel");

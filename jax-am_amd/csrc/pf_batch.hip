@@ -206,7 +206,7 @@ int rebuild_work(pf_batch* b) {
     const StepDev& a = sh.a;
     tiles[s] = SlotTiles{a.tiles_x, a.tiles_y, a.tiles_z, a.zc, a.zs, a.zsplit};
     const BatchClass& k = b->classes[sh.cls];
-    const long long items = !k.quads              ? (long long)a.tiles_x * a.tiles_y * a.tiles_z
+    const long long items = !k.quads                  ? (long long)a.tiles_x * a.tiles_y * a.tiles_z
                             : quad_fits(k.dtype, k.k) ? 8LL * a.tiles_y * a.tiles_z
                                                       : sh.charge;
     if (items >= (1LL << 31)) return fail(PF_E_ARG, "instance too large");
