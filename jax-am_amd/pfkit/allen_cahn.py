@@ -146,10 +146,11 @@ def explicit_euler(state_pre, t_crt, f, ode_params):
 def rk4(state_pre, t_crt, f, ode_params):
     """allen_cahn.py:90-103 (classical RK4): four stage kernels that form the combinations of the
     right-hand sides as they compute them (pf_rk4), or four pf_rhs evaluations where f is not a
-    plain StateRHS or has more orientations than those kernels take."""
+    plain StateRHS, has more orientations than those kernels take, or the state is tracked by autograd
+    (which then follows the combination of the stages)."""
     y_prev, t_prev = state_pre
     y_prev = f.check_state(y_prev)
-    if type(f) is StateRHS:
+    if type(f) is StateRHS and not y_prev.requires_grad:
         T, = ode_params
         y = f.rk4_step(y_prev, T, t_prev, t_crt)
         if y is not None:
