@@ -6,7 +6,8 @@
 //     so a captured graph stays valid while instances come and go.
 //   - Instances are grouped into classes (dtype, K, anisotropy, tile shape).  Each
 //     class has a device-resident work list of (slot, tile) items walked by one
-//     persistent launch per step with a fixed grid.
+//     persistent launch per step with a fixed grid; in a captured block of steps the classes (or the parts
+//     of a lone large one) run on branches of the graph.
 //   - A class whose instances together leave the GPU short of workgroups runs shorter marches than its
 //     instances ask for, or the march of channel groups (rebuild_work).
 //   - `chunk` steps (launches of the classes that have work, an advance per block) are captured
@@ -88,7 +89,6 @@ struct BatchClass {
   int dtype, k, aniso, tile;
   const StepEntry* entry;  // tile shape, null for K without tiled kernels
   bool quads;              // the class runs the march of channel groups (always for a null entry)
-  int off;    // offset of this class's work list in d_work
   int count;  // host copy of the work-item count
   int users;  // slots in this class; a class without users is retired and its index reused
 };
@@ -115,24 +115,34 @@ struct pf_batch {
   BatchSlot* d_slots = nullptr;
   WorkItem* d_work = nullptr;
   size_t work_cap = 0;     // items that d_work holds (at least max_tiles)
-  int2* d_info = nullptr;  // per class (work-list offset, count)
+  int2* d_info = nullptr;  // per class (work-list offset, count), then those of a lone class's parts
   SlotTiles* d_tiles = nullptr;
   std::vector<SlotHost> slots;
   std::vector<BatchClass> classes;
   bool work_dirty = false;
+  int parts = 1;  // that a lone class's instances are dealt to (rebuild_work)
   struct Graph {
     int chunk;
     unsigned long long mask, quads;  // classes with work, and those of them on channel groups
+    int parts;                       // of a lone class
     hipGraph_t def;
     hipGraphExec_t exec;
   };
   static constexpr int kMaxGraphs = 16;
   std::vector<Graph> graphs;  // most recently used last
+  static constexpr int kSide = 2;  // streams that a captured block of steps forks to (launch_steps)
+  hipStream_t side[kSide] = {};
+  hipEvent_t forked = nullptr, joined[kSide] = {};
   std::mutex mu;
 };
 
 namespace {
 
+// Values (cells x orientations) from which a lone tiled class's launches are split over the branches: 21 million of
+// eight 64x64x32 48.2 -> 44.7 us a step; below, three of 36x36x30 (2.3 million) 14.3 -> 16.0, twelve of 32^3, K = 10
+// (3.9 million) 17.6 -> 18.9.  On channel groups a split loses at any size measured (50x50x34, K = 33 38 -> 42).
+constexpr long long kSplitValues = 12000000;
+constexpr int kForkSteps = 4;  // steps of a block from which its launches fork (launch_steps)
 constexpr int kBatchQuads = 1024;  // workgroups of the batched march of channel groups on 256 CUs
 
 void drop_graphs(pf_batch* b) {
@@ -197,8 +207,18 @@ void tile_class(pf_batch* b, int c) {
 int rebuild_work(pf_batch* b) {
   for (size_t c = 0; c < b->classes.size(); ++c)
     if (b->classes[c].users > 0) tile_class(b, (int)c);
-  // pack each class's work items contiguously, in slot order
-  std::vector<std::vector<WorkItem>> per(b->classes.size());
+  // pack each class's work items contiguously, in slot order; of a lone class, each part's: a slot goes to the
+  // part with the fewest items so far
+  int live = 0, used = 0;
+  for (const BatchClass& k : b->classes) live += k.users > 0;
+  long long values = 0;
+  for (const SlotHost& sh : b->slots)
+    if (sh.used && !b->classes[sh.cls].quads) {
+      used += 1;
+      values += (long long)sh.a.nz * sh.a.ny * sh.a.nx * b->classes[sh.cls].k;
+    }
+  b->parts = live == 1 && values >= kSplitValues ? std::min(used, 1 + pf_batch::kSide) : 1;
+  std::vector<std::vector<WorkItem>> per(pf_batch::kMaxClasses + 1 + pf_batch::kSide);
   std::vector<SlotTiles> tiles(b->max_inst, SlotTiles{0, 0, 0, 0, 0, 0});
   for (int s = 0; s < b->max_inst; ++s) {
     const SlotHost& sh = b->slots[s];
@@ -210,16 +230,24 @@ int rebuild_work(pf_batch* b) {
                             : quad_fits(k.dtype, k.k) ? 8LL * a.tiles_y * a.tiles_z
                                                       : sh.charge;
     if (items >= (1LL << 31)) return fail(PF_E_ARG, "instance too large");
-    for (int t = 0; t < (int)items; ++t) per[sh.cls].push_back(WorkItem{s, t, sh.path, 0});
+    int to = b->parts > 1 ? pf_batch::kMaxClasses : sh.cls;
+    for (int p = 1; p < b->parts; ++p)
+      if (per[pf_batch::kMaxClasses + p].size() < per[to].size()) to = pf_batch::kMaxClasses + p;
+    for (int t = 0; t < (int)items; ++t) per[to].push_back(WorkItem{s, t, sh.path, 0});
   }
   std::vector<WorkItem> all;
-  std::vector<int2> info(pf_batch::kMaxClasses, make_int2(0, 0));
-  for (size_t c = 0; c < b->classes.size(); ++c) {
-    b->classes[c].off = (int)all.size();
-    b->classes[c].count = (int)per[c].size();
+  std::vector<int2> info(per.size());
+  for (size_t c = 0; c < per.size(); ++c) {
+    if (c < b->classes.size()) b->classes[c].count = (int)per[c].size();
     info[c] = make_int2((int)all.size(), (int)per[c].size());
     all.insert(all.end(), per[c].begin(), per[c].end());
   }
+  if (b->parts > 1)  // the class's own entry spans its parts, which lie one after the other
+    for (size_t c = 0; c < b->classes.size(); ++c)
+      if (b->classes[c].users > 0) {
+        b->classes[c].count = (int)all.size();
+        info[c] = make_int2(0, (int)all.size());
+      }
   hipError_t e = hipSuccess;
   if (all.size() > b->work_cap) {
     // more items than max_tiles, by which slots are charged as they asked to be tiled: a longer list;
@@ -267,22 +295,53 @@ unsigned long long quad_mask(const pf_batch* b) {
   return m;
 }
 
-// `steps` steps of every class with work, in blocks of up to kPlan with an advance after each.
-int launch_steps(pf_batch* b, int steps) {
+// `steps` steps of every class with work, in blocks of up to kPlan with an advance after each.  The classes' slots
+// have nothing in common but the tables, which only the advance writes: with `fork` (a capture) a block's
+// launches of different classes, or of a lone class's parts, run on branches of the graph, each step after step,
+// and their tails and latencies overlap.  us a step, on one stream -> forked: eighteen requests of 36x36x30 to
+// 72x72x40 in six classes 87 -> 60, 64 instances of 32^3 to 128x128x64 4.41e11 -> 5.06e11 updates/s; a lone class
+// of K = 20: eight of 64x64x32 in FP32 48.2 -> 44.7, eight of 72x72x40 in BF16 51.5 -> 43.6, four in FP64 133 -> 108.  The fork and the
+// join take about 13 us a block: three classes of one 32^3 instance each 26.9 -> 46.3 in blocks of one step, 22.2 -> 30.3 of
+// two, 19.8 -> 18.3 of four, 18.9 -> 15.3 of eight; hence kForkSteps.  More branches than three gained nothing.
+int launch_steps(pf_batch* b, int steps, bool fork) {
   const BatchView v{b->d_desc, b->d_dyn, b->d_slots, b->d_work, b->d_info, b->max_inst};
+  struct Launch {
+    int cls, info;  // class, and which entry of d_info holds its items
+  };
+  std::vector<Launch> whole, parts;
+  for (size_t c = 0; c < b->classes.size(); ++c) {
+    if (b->classes[c].count == 0) continue;
+    whole.push_back(Launch{(int)c, (int)c});
+    for (int p = 0; p < b->parts; ++p)
+      parts.push_back(Launch{(int)c, b->parts > 1 ? pf_batch::kMaxClasses + p : (int)c});
+  }
   for (int done = 0; done < steps;) {
     const int n = std::min(kPlan, steps - done);
+    const bool forked = fork && n >= kForkSteps;
+    const std::vector<Launch>& live = forked ? parts : whole;
+    const int branches = forked ? std::max(1, std::min((int)live.size(), 1 + pf_batch::kSide)) : 1;
+    hipError_t e = hipSuccess;
+    if (branches > 1) e = hipEventRecord(b->forked, b->stream);
+    for (int s = 1; s < branches && e == hipSuccess; ++s) e = hipStreamWaitEvent(b->side[s - 1], b->forked, 0);
+    if (e != hipSuccess) return hip_fail(e, "pf_batch fork");
     for (int i = 0; i < n; ++i) {
-      for (size_t c = 0; c < b->classes.size(); ++c) {
-        const BatchClass& k = b->classes[c];
-        if (k.count == 0) continue;
+      for (size_t l = 0; l < live.size(); ++l) {
+        const BatchClass& k = b->classes[live[l].cls];
+        // (workgroups: tiled classes 1024 / 2048 / 4096 / 8192: c3 4.73 / 4.90 / 5.06 / 5.10e11 updates/s, two of
+        // 256x256x64 271 / 279 / 267 / 265 us, but six small classes 59.9 / 59.3 / 60.6 / 64.7 us)
         const BatchLaunch fn = k.quads ? generic_batch(k.dtype, k.k, k.aniso != 0) : k.entry->batch;
-        hipError_t e = fn(v, (int)c, i, k.quads ? 2048 : 1024, k.k, b->stream);
+        const int s = (int)(l % branches);
+        e = fn(v, live[l].info, i, k.quads ? 2048 : 4096, k.k, s ? b->side[s - 1] : b->stream);
         if (e != hipSuccess) return hip_fail(e, "pf_batch step launch");
       }
     }
+    for (int s = 1; s < branches && e == hipSuccess; ++s) {
+      e = hipEventRecord(b->joined[s - 1], b->side[s - 1]);
+      if (e == hipSuccess) e = hipStreamWaitEvent(b->stream, b->joined[s - 1], 0);
+    }
+    if (e != hipSuccess) return hip_fail(e, "pf_batch join");
     advance_kernel<<<(b->max_inst + 7) / 8, 8 * kPlan, 0, b->stream>>>(b->d_desc, b->d_slots, b->d_dyn, b->max_inst, n);
-    hipError_t e = hipGetLastError();
+    e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "pf_batch advance launch");
     done += n;
   }
@@ -308,7 +367,8 @@ void drop_graphs_of_class(pf_batch* b, int c) {
 int get_graph(pf_batch* b, int chunk, hipGraphExec_t* out) {
   const unsigned long long mask = active_mask(b), quads = quad_mask(b);
   for (size_t i = 0; i < b->graphs.size(); ++i) {
-    if (b->graphs[i].chunk == chunk && b->graphs[i].mask == mask && b->graphs[i].quads == quads) {
+    if (b->graphs[i].chunk == chunk && b->graphs[i].mask == mask && b->graphs[i].quads == quads &&
+        b->graphs[i].parts == b->parts) {
       pf_batch::Graph g = b->graphs[i];
       b->graphs.erase(b->graphs.begin() + i);
       b->graphs.push_back(g);
@@ -318,7 +378,7 @@ int get_graph(pf_batch* b, int chunk, hipGraphExec_t* out) {
   }
   hipError_t e = hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) return hip_fail(e, "hipStreamBeginCapture");
-  const int rc = launch_steps(b, chunk);
+  const int rc = launch_steps(b, chunk, true);
   hipGraph_t g = nullptr;
   e = hipStreamEndCapture(b->stream, &g);
   if (rc) {
@@ -339,7 +399,7 @@ int get_graph(pf_batch* b, int chunk, hipGraphExec_t* out) {
     (void)hipGraphDestroy(b->graphs.front().def);
     b->graphs.erase(b->graphs.begin());
   }
-  b->graphs.push_back(pf_batch::Graph{chunk, mask, quads, g, ex});
+  b->graphs.push_back(pf_batch::Graph{chunk, mask, quads, b->parts, g, ex});
   *out = ex;
   return PF_OK;
 }
@@ -363,12 +423,17 @@ pf_batch_t* pf_batch_create(int32_t max_instances, int32_t max_tiles, void* stre
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_dyn, sizeof(StepDyn) * kPlan * max_instances);
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_slots, sizeof(BatchSlot) * max_instances);
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_work, sizeof(WorkItem) * max_tiles);
-  if (e == hipSuccess) e = hipMalloc((void**)&b->d_info, sizeof(int2) * pf_batch::kMaxClasses);
+  if (e == hipSuccess) e = hipMalloc((void**)&b->d_info, sizeof(int2) * (pf_batch::kMaxClasses + 1 + pf_batch::kSide));
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_tiles, sizeof(SlotTiles) * max_instances);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&b->forked, hipEventDisableTiming);
+  for (int s = 0; s < pf_batch::kSide && e == hipSuccess; ++s) {
+    e = hipStreamCreateWithFlags(&b->side[s], hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&b->joined[s], hipEventDisableTiming);
+  }
   if (e == hipSuccess) {
     std::vector<BatchSlot> z(max_instances);
     memset(z.data(), 0, z.size() * sizeof(BatchSlot));
-    std::vector<int2> zc(pf_batch::kMaxClasses, make_int2(0, 0));
+    std::vector<int2> zc(pf_batch::kMaxClasses + 1 + pf_batch::kSide, make_int2(0, 0));
     e = hipMemcpyAsync(b->d_slots, z.data(), z.size() * sizeof(BatchSlot), hipMemcpyHostToDevice, b->stream);
     if (e == hipSuccess)
       e = hipMemcpyAsync(b->d_info, zc.data(), zc.size() * sizeof(int2), hipMemcpyHostToDevice, b->stream);
@@ -386,6 +451,11 @@ void pf_batch_destroy(pf_batch_t* b) {
   if (!b) return;
   if (b->stream) (void)hipStreamSynchronize(b->stream);
   drop_graphs(b);
+  if (b->forked) (void)hipEventDestroy(b->forked);
+  for (int s = 0; s < pf_batch::kSide; ++s) {
+    if (b->joined[s]) (void)hipEventDestroy(b->joined[s]);
+    if (b->side[s]) (void)hipStreamDestroy(b->side[s]);
+  }
   if (b->d_desc) (void)hipFree(b->d_desc);
   if (b->d_dyn) (void)hipFree(b->d_dyn);
   if (b->d_slots) (void)hipFree(b->d_slots);
@@ -447,7 +517,7 @@ int pf_batch_add(pf_batch_t* b, const pf_batch_inst_t* inst) {
   }
   if (cls < 0) {
     // a new class takes a retired index (its graphs were dropped when it retired) or a new one
-    const BatchClass nc{inst->dtype, inst->p.num_oris, (int)aniso, tile, e, !e, 0, 0, 0};
+    const BatchClass nc{inst->dtype, inst->p.num_oris, (int)aniso, tile, e, !e, 0, 0};
     if (free_cls >= 0) {
       b->classes[free_cls] = nc;
       cls = free_cls;
@@ -518,7 +588,7 @@ int pf_batch_run(pf_batch_t* b, int32_t steps, int32_t chunk) {
       if (e != hipSuccess) return hip_fail(e, "hipGraphLaunch");
     }
   }
-  return launch_steps(b, steps - done);
+  return launch_steps(b, steps - done, false);
 }
 
 int pf_batch_status(pf_batch_t* b, int32_t* steps_left, double* t, int32_t* parity, int32_t n) {

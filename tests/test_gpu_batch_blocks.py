@@ -54,6 +54,32 @@ def test_a_class_changes_its_kernel_as_instances_come_and_go(cuda, dtype, k):
     eng.close()
 
 
+@pytest.mark.parametrize("ks,dtype,chunk", [((6, 9, 12, 27, 16), "float32", 8), ((6, 9, 12, 27, 16), "bfloat16", 3),
+                                            ((10, 13), "float64", 12), ((20,), "float32", 4), ((20,), "float32", 3),
+                                            ((20,), "bfloat16", 16), ((16,), "float64", 5)])
+def test_classes_and_parts_that_run_side_by_side(cuda, ks, dtype, chunk):
+    """More classes than branches, fewer, and a lone class large enough to be split (four instances of uneven size,
+    then two, then one): replays with eager steps and host reads between, each instance bitwise its own run."""
+    if len(ks) > 1:
+        W = [_make(j, 30 + 3 * j, 26, 12, k, dtype, 80) for j, k in enumerate(ks + ks[:2])]
+    else:
+        W = [_make(j, 96 + 8 * j, 90, 25, ks[0], dtype, 80) for j in range(4)]
+    eng = BatchEngine(max_instances=8)
+    slots = [eng.add(w.instance()) for w in W]
+    done = 0
+    for rest in (1, 0, 2):
+        eng.run(2 * chunk + rest, chunk)
+        done += 2 * chunk + rest
+        par = eng.status()[2]
+        for w, s in zip(W, slots):
+            assert torch.equal(eng.state(s, par[s]), _solo(w, min(done, 80)))
+        if rest < 1 or len(ks) == 1:
+            for s in slots[len(slots) // 2:]:
+                eng.remove(s)
+            slots = slots[:len(slots) // 2]
+    eng.close()
+
+
 def test_more_work_items_than_max_tiles(cuda):
     """Slots are charged as they asked to be tiled; shorter marches and channel groups make more work items than that,
     and the work list grows (between replays of graphs that held the shorter one)."""
