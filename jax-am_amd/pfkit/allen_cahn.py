@@ -18,7 +18,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .config import PACKED_KEYS, make_params, with_defaults
+from .config import make_params, with_defaults
 from .laser import LASERS
 
 DTYPES = {"float64": torch.float64, "float32": torch.float32, "bfloat16": torch.bfloat16,
@@ -51,28 +51,14 @@ class StateRHS:
                                     device=self.device) if self.aniso else None
         self.pf_dtype = _lib.TORCH_TO_PF[self.dtype]
         self._T_keep = None
-        self._packed = (None, None, None)
         _lib.load()
 
     # ---- temperature argument
-    def _params(self, laser=None):
-        """pf_params_t of the current pf_args and h_xyz with this laser descriptor: a copy of the struct
-        packed last while their values are the same (packing its fields takes longer than a launch)."""
-        values, h, p0 = self._packed
-        now = PACKED_KEYS(self.pf_args)
-        if values != now or h != self.h_xyz:
-            p0 = make_params(self.pf_args, self.h_xyz, None)
-            self._packed = (now, self.h_xyz, p0)
-        p = _lib.ParamsT.from_buffer_copy(p0)
-        if laser is not None:
-            laser.fill(p.laser)
-        return p
-
     def params_for(self, T):
         """pf_params_t and the T device pointer for ode_params[0] = T."""
         if isinstance(T, LASERS):
-            return self._params(T), None
-        p = self._params()
+            return make_params(self.pf_args, self.h_xyz, T), None
+        p = make_params(self.pf_args, self.h_xyz, None)
         Tt = torch.as_tensor(T, device=self.device)
         if Tt.dtype not in (torch.float64, torch.float32):
             Tt = Tt.to(torch.float64)

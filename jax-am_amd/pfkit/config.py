@@ -16,7 +16,9 @@ liquid_shift       1.0      allen_cahn.py:124
 anisotropy         0.0      pf_params.yaml
 =================  =======  =========================================
 """
+import ctypes
 import math
+import struct
 from operator import itemgetter
 
 import yaml
@@ -24,11 +26,6 @@ import yaml
 from . import _lib
 
 HARD_CODED = dict(gamma=1.0, T_clip=2000.0, zeta_sharpness=1e10, force_liquid=False, liquid_shift=1.0)
-
-
-# the values that make_params packs, as a tuple
-PACKED_KEYS = itemgetter("Nz", "Ny", "Nx", "num_oris", "m_g", "gamma", "kappa_g", "ad_hoc", "L0", "Qg", "gas_const",
-                         "T_liquidus", "T_clip", "zeta_sharpness", "anisotropy", "force_liquid", "liquid_shift")
 
 
 def yaml_parse(path):
@@ -71,27 +68,33 @@ def stable_dt(pf_args, h_xyz, fraction=0.2, c_local=None):
     return fraction * dt_max, dt_max, c
 
 
+# The values of pf_params_t in the order of its fields, without its mesh size and laser, and the layout up to its laser.
+_VALUES = itemgetter("Nz", "Ny", "Nx", "num_oris", "m_g", "gamma", "kappa_g", "ad_hoc", "L0", "Qg", "gas_const",
+                     "T_liquidus", "T_clip", "zeta_sharpness", "anisotropy", "force_liquid", "liquid_shift")
+_HEAD = struct.Struct("@4i14dixxxxd")
+_REST = bytes(ctypes.sizeof(_lib.ParamsT) - _HEAD.size)
+assert _HEAD.size == _lib.ParamsT.laser.offset
+
+
 def make_params(pf_args, h_xyz, laser=None):
-    """Pack pf_args (+ a laser descriptor) into the C struct pf_params_t."""
-    a = with_defaults(pf_args)
-    p = _lib.ParamsT()
-    p.nz, p.ny, p.nx = int(a["Nz"]), int(a["Ny"]), int(a["Nx"])
-    p.num_oris = int(a["num_oris"])
-    for d in range(3):
-        p.h[d] = float(h_xyz[d])
-    p.m_g = float(a["m_g"])
-    p.gamma = float(a["gamma"])
-    p.kappa_g = float(a["kappa_g"])
-    p.ad_hoc = float(a["ad_hoc"])
-    p.L0 = float(a["L0"])
-    p.Qg = float(a["Qg"])
-    p.gas_const = float(a["gas_const"])
-    p.T_liquidus = float(a["T_liquidus"])
-    p.T_clip = float(a["T_clip"])
-    p.zeta_sharpness = float(a["zeta_sharpness"])
-    p.anisotropy = float(a["anisotropy"])
-    p.force_liquid = 1 if a["force_liquid"] else 0
-    p.liquid_shift = float(a["liquid_shift"])
+    """Pack pf_args (+ a laser descriptor) into the C struct pf_params_t.
+
+    Every call reads the values that pf_args holds then: they may be arrays or tensors that are changed in
+    place.  Packed by one call of struct (a small step is launched every few microseconds)."""
+    try:
+        if type(pf_args) is not dict:
+            raise KeyError
+        nz, ny, nx, k, *v, force, shift = _VALUES(pf_args)
+    except KeyError:
+        nz, ny, nx, k, *v, force, shift = _VALUES(with_defaults(pf_args))
+    force = 1 if force else 0
+    try:
+        head = _HEAD.pack(nz, ny, nx, k, h_xyz[0], h_xyz[1], h_xyz[2], *v, force, shift)
+    except (struct.error, TypeError):
+        # values of other types (text from a yaml file, sizes as floats); sizes to 32 bits as ctypes takes them
+        size = [(int(n) + 2 ** 31) % 2 ** 32 - 2 ** 31 for n in (nz, ny, nx, k)]
+        head = _HEAD.pack(*size, *(float(x) for x in (h_xyz[0], h_xyz[1], h_xyz[2], *v)), force, float(shift))
+    p = _lib.ParamsT.from_buffer_copy(head + _REST)
     if laser is not None:
         laser.fill(p.laser)
     else:

@@ -39,9 +39,10 @@ class Rosenthal:
     def fill(self, L):
         L.model = _lib.PF_T_ROSENTHAL
         L.T_ambient = self.T_ambient
-        for d in range(3):
-            L.pos0[d] = self.pos0[d]
-            L.dir[d] = self.dir[d]
+        p, d = L.pos0, L.dir
+        for i in range(3):
+            p[i] = self.pos0[i]
+            d[i] = self.dir[i]
         L.vel = self.vel
         L.Q, L.kappa_T, L.alpha, L.T_cap = self.Q, self.kappa_T, self.alpha, self.T_cap
 
@@ -65,9 +66,10 @@ class Gaussian:
     def fill(self, L):
         L.model = _lib.PF_T_GAUSSIAN
         L.T_ambient = self.T_ambient
-        for d in range(3):
-            L.pos0[d] = self.pos0[d]
-            L.dir[d] = self.dir[d]
+        p, d = L.pos0, L.dir
+        for i in range(3):
+            p[i] = self.pos0[i]
+            d[i] = self.dir[i]
         L.vel = self.vel
         L.dT_peak, L.sigma_xy, L.sigma_z = self.dT_peak, self.sigma_xy, self.sigma_z
 
