@@ -220,6 +220,20 @@ bool small_step(int dtype, int k, long long cells) {
   return quad_threads(dtype, k, cells) <= most;
 }
 
+// Whether a step's tiles go to the XCDs by whole rows (tile_coords): where the XCD with the most rows needs no
+// more fillings than an even share would, `held` workgroups being resident on the GPU at once, and none
+// stays empty.  Sharing an L2 along a row is worth 3 to 7 % (us a step, rows against even shares: 203x197x59,
+// K = 20, FP32 85.0/91.4, 300x100x80 85.3/91.6, 100x300x40 48.3/51.3); a filling more costs far more than
+// that (320x72x48, 36 rows of 40 tiles, 192 held per XCD: 54.9/44.8; 200x56x64, K = 17, 77 rows of 13, 128 held:
+// 35.8/33.9), and so do XCDs without work (4096x32x1, K = 20, 4 rows: 16.5/10.4).
+static int deal_rows(const StepDev& a, int held) {
+  const long long rows = (long long)a.tiles_y * a.tiles_z;
+  if (rows < 8) return 0;
+  const long long most = (rows + 7) / 8 * a.tiles_x, even = (rows * a.tiles_x + 7) / 8;
+  const long long cap = held >= 8 ? held / 8 : 1;
+  return (most + cap - 1) / cap == (even + cap - 1) / cap;
+}
+
 static const StepEntry* choose_step(int dtype, int k, bool aniso, long long cells) {
   if (small_step(dtype, k, cells)) return nullptr;
   const bool odd = k % 2 != 0;
@@ -492,7 +506,8 @@ static int plan_step(const pf_params_t* p, int dtype, const void* T_dev, const v
     const long long cols = (long long)((p->nx + e->tx - 1) / e->tx) * ((p->ny + e->ty - 1) / e->ty);
     if ((zchunk & 0xffff) == 0) zchunk |= fill_zchunk(p->nz, cols, held_workgroups(e, false));
     set_tiles(a, e->tx, e->ty, zchunk);
-    if (tile_launch(a.tiles_x, a.tiles_y, a.tiles_z) >= (1LL << 31)) return fail(PF_E_ARG, "too many tiles");
+    a.rows = deal_rows(a, held_workgroups(e, false));
+    if (tile_launch(a) >= (1LL << 31)) return fail(PF_E_ARG, "too many tiles");
     fn = e->step;
   } else {
     if (!grid_ok(n, 1)) return fail(PF_E_ARG, "grid too large for the generic kernel");

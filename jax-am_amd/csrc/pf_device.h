@@ -101,7 +101,8 @@ struct StepDev {
   int nz, ny, nx, k;
   int tiles_x, tiles_y, tiles_z, zc;
   int zs, zsplit;      // planes [0, zsplit) in chunks of zs, [zsplit, nz) in chunks of zc (zsplit 0: no tail)
-  int tmodel, t_f64, force_liquid, pad0;
+  int tmodel, t_f64, force_liquid;
+  int rows;            // 1: a step's tiles go to the XCDs by whole rows (tile_coords)
   float ihx2f, ihy2f, ihz2f, Bf;          // FP32 copies of ihx2, ihy2, ihz2, B
   double hx, hy, hz;
   double ihx2, ihy2, ihz2;
@@ -1512,29 +1513,36 @@ __device__ __forceinline__ void generic_cell(const StepDev& a, const StepDyn& dy
   }
 }
 
-// Tile order of a launch: rows of tiles, layer by layer of z-chunks from the top of the domain down.
-// Workgroups are dispatched in index order and dealt round-robin to the 8 XCDs, so the top layer, where a
+// Tile order of a launch: layers of z-chunks from the top of the domain down.  Workgroups are
+// dispatched in index order and dealt round-robin to the 8 XCDs, so the top layer, where a
 // surface heat source makes cells hot and the per-cell FP64 path slow, starts first and the
-// cheaper layers below fill in behind it.  Workgroup t takes the next tile of row 8m + (t mod 8), the rows of
-// all layers counted together: every XCD then walks whole rows of tiles, so the x-neighbours of a tile
-// (whose halo columns it re-reads) run on the same XCD and share its L2, and the XCDs' shares
-// differ by one row at most.  (Dealt tile by tile where a layer's rows did not divide by 8: 203x197x59,
-// K = 20, FP32 8x8 lane pairs 94.6 us, by rows 85.8; 150x140x50 46.1 and 38.6.)  The rows are padded to a multiple of 8: false for a
-// workgroup past the last one.
-__host__ __device__ inline long long tile_launch(int tiles_x, int tiles_y, int tiles_z) {
-  return ((long long)tiles_y * tiles_z + 7) / 8 * 8 * tiles_x;
+// cheaper layers below fill in behind it.  Two ways to deal a layer:
+//   a.rows: workgroup t takes the next tile of row 8m + (t mod 8), the rows of all layers counted
+//     together: every XCD walks whole rows of tiles, so the x-neighbours of a tile (whose halo columns it
+//     re-reads) run on the same XCD and share its L2.  The rows are padded to a multiple of 8 (false for a
+//     workgroup past the last one); an XCD's share is whole rows, up to one row more than an even share;
+//   else as item_coords deals an instance's tiles, no padding, shares that differ by one tile.
+// deal_rows (pf_abi.hip) chooses.
+__host__ __device__ inline long long tile_launch(const StepDev& a) {
+  const long long rows = (long long)a.tiles_y * a.tiles_z;
+  return (a.rows ? (rows + 7) / 8 * 8 : rows) * a.tiles_x;
 }
-__device__ __forceinline__ bool tile_coords(int t, int tiles_x, int tiles_y, int tiles_z, int& tx, int& ty, int& tz) {
-  const int i = t >> 3, m = i / tiles_x;
-  tx = i - m * tiles_x;
-  const int row = 8 * m + (t & 7), layer = row / tiles_y;
-  ty = row - layer * tiles_y;
-  tz = tiles_z - 1 - layer;
+__device__ __forceinline__ void item_coords(int t, int tiles_x, int tiles_y, int tiles_z, int& tx, int& ty, int& tz);
+__device__ __forceinline__ bool tile_coords(const StepDev& a, int t, int& tx, int& ty, int& tz) {
+  if (!a.rows) {
+    item_coords(t, a.tiles_x, a.tiles_y, a.tiles_z, tx, ty, tz);
+    return true;
+  }
+  const int i = t >> 3, m = i / a.tiles_x;
+  tx = i - m * a.tiles_x;
+  const int row = 8 * m + (t & 7), layer = row / a.tiles_y;
+  ty = row - layer * a.tiles_y;
+  tz = a.tiles_z - 1 - layer;
   return tz >= 0;
 }
 
-// The same for a work item of the batch engine: an instance's layers follow each other without padding, and
-// only layers whose rows divide by 8 are dealt by rows (64 instances of 32^3 to 128x128x64: 4.27e11 updates/s,
+// Tile t of a grid whose layers follow each other without padding (a work item of the batch engine, a launch
+// that is not dealt by rows): whole rows to an XCD in layers whose rows divide by 8, else x fastest, then y (64 instances of 32^3 to 128x128x64: 4.27e11 updates/s,
 // with every instance dealt by padded rows 4.14e11).
 __device__ __forceinline__ void item_coords(int t, int tiles_x, int tiles_y, int tiles_z, int& tx, int& ty, int& tz) {
   const int nl = tiles_x * tiles_y;

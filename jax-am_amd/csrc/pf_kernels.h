@@ -84,7 +84,7 @@ __global__ __launch_bounds__(TX* TY* H) __attribute__((amdgpu_waves_per_eu(H + 1
   __shared__ __attribute__((aligned(16))) TC ax[ANISO ? G::AXN : 4];
   __shared__ ZTab zt;
   int tx, ty, tz;
-  if (!tile_coords(blockIdx.x, a.tiles_x, a.tiles_y, a.tiles_z, tx, ty, tz)) return;
+  if (!tile_coords(a, blockIdx.x, tx, ty, tz)) return;
   march_tile<K, TS, ANISO, TX, TY, H>(a, d, tx, ty, tz, smem, stage, ax, &zt);
 }
 
@@ -129,7 +129,7 @@ struct StepEntry {
 
 template <int K, class TS, bool ANISO, int TX, int TY, int H>
 hipError_t launch_step(const StepDev& a, const StepDyn& d, hipStream_t s) {
-  const unsigned n = (unsigned)tile_launch(a.tiles_x, a.tiles_y, a.tiles_z);
+  const unsigned n = (unsigned)tile_launch(a);
   step_kernel<K, TS, ANISO, TX, TY, H><<<dim3(n), dim3(TX * TY * H), 0, s>>>(a, d);
   return hipGetLastError();
 }
