@@ -16,7 +16,6 @@ liquid_shift       1.0      allen_cahn.py:124
 anisotropy         0.0      pf_params.yaml
 =================  =======  =========================================
 """
-import ctypes
 import math
 import struct
 from operator import itemgetter
@@ -72,7 +71,6 @@ def stable_dt(pf_args, h_xyz, fraction=0.2, c_local=None):
 _VALUES = itemgetter("Nz", "Ny", "Nx", "num_oris", "m_g", "gamma", "kappa_g", "ad_hoc", "L0", "Qg", "gas_const",
                      "T_liquidus", "T_clip", "zeta_sharpness", "anisotropy", "force_liquid", "liquid_shift")
 _HEAD = struct.Struct("@4i14dixxxxd")
-_REST = bytes(ctypes.sizeof(_lib.ParamsT) - _HEAD.size)
 assert _HEAD.size == _lib.ParamsT.laser.offset
 
 
@@ -84,17 +82,19 @@ def make_params(pf_args, h_xyz, laser=None):
     try:
         if type(pf_args) is not dict:
             raise KeyError
-        nz, ny, nx, k, *v, force, shift = _VALUES(pf_args)
+        values = _VALUES(pf_args)
     except KeyError:
-        nz, ny, nx, k, *v, force, shift = _VALUES(with_defaults(pf_args))
+        values = _VALUES(with_defaults(pf_args))
+    nz, ny, nx, k, m_g, gamma, kappa_g, ad_hoc, L0, Qg, gas_const, T_l, T_clip, sharp, aniso, force, shift = values
     force = 1 if force else 0
+    p = _lib.ParamsT()
     try:
-        head = _HEAD.pack(nz, ny, nx, k, h_xyz[0], h_xyz[1], h_xyz[2], *v, force, shift)
+        _HEAD.pack_into(p, 0, nz, ny, nx, k, h_xyz[0], h_xyz[1], h_xyz[2], m_g, gamma, kappa_g, ad_hoc, L0, Qg,
+                        gas_const, T_l, T_clip, sharp, aniso, force, shift)
     except (struct.error, TypeError):
         # values of other types (text from a yaml file, sizes as floats); sizes to 32 bits as ctypes takes them
         size = [(int(n) + 2 ** 31) % 2 ** 32 - 2 ** 31 for n in (nz, ny, nx, k)]
-        head = _HEAD.pack(*size, *(float(x) for x in (h_xyz[0], h_xyz[1], h_xyz[2], *v)), force, float(shift))
-    p = _lib.ParamsT.from_buffer_copy(head + _REST)
+        _HEAD.pack_into(p, 0, *size, *(float(x) for x in (h_xyz[0], h_xyz[1], h_xyz[2], *values[4:15])), force, float(shift))
     if laser is not None:
         laser.fill(p.laser)
     else:

@@ -6,11 +6,13 @@ one of these descriptors instead lets the kernel evaluate T at each cell centroi
 (FP64) with no temperature array in memory.  The reference's array form is still
 accepted by ``PFSolver.stepper`` (PF_T_BUFFER).
 """
+import struct
 from dataclasses import dataclass
 from typing import Tuple
 
 from . import _lib
 
+_LASER = struct.Struct("@2i18d")  # pf_laser_t; one call sets all fields (a step is launched every few microseconds)
 
 @dataclass
 class Rosenthal:
@@ -37,14 +39,9 @@ class Rosenthal:
                    vel=0.6 * pf_args["domain_x"] / pf_args["t_OFF"], T_ambient=pf_args["T_ambient"])
 
     def fill(self, L):
-        L.model = _lib.PF_T_ROSENTHAL
-        L.T_ambient = self.T_ambient
-        p, d = L.pos0, L.dir
-        for i in range(3):
-            p[i] = self.pos0[i]
-            d[i] = self.dir[i]
-        L.vel = self.vel
-        L.Q, L.kappa_T, L.alpha, L.T_cap = self.Q, self.kappa_T, self.alpha, self.T_cap
+        p, d = self.pos0, self.dir
+        _LASER.pack_into(L, 0, _lib.PF_T_ROSENTHAL, 0, self.T_ambient, p[0], p[1], p[2], d[0], d[1], d[2], self.vel,
+                         self.Q, self.kappa_T, self.alpha, self.T_cap, 0, 0, 0, 0, 0, 0)
 
     def as_dict(self):
         return dict(model="rosenthal", pos0=self.pos0, vel=self.vel, Q=self.Q, alpha=self.alpha,
@@ -64,14 +61,9 @@ class Gaussian:
     dir: Tuple[float, float, float] = (1.0, 0.0, 0.0)
 
     def fill(self, L):
-        L.model = _lib.PF_T_GAUSSIAN
-        L.T_ambient = self.T_ambient
-        p, d = L.pos0, L.dir
-        for i in range(3):
-            p[i] = self.pos0[i]
-            d[i] = self.dir[i]
-        L.vel = self.vel
-        L.dT_peak, L.sigma_xy, L.sigma_z = self.dT_peak, self.sigma_xy, self.sigma_z
+        p, d = self.pos0, self.dir
+        _LASER.pack_into(L, 0, _lib.PF_T_GAUSSIAN, 0, self.T_ambient, p[0], p[1], p[2], d[0], d[1], d[2], self.vel,
+                         0, 0, 0, 0, self.dT_peak, self.sigma_xy, self.sigma_z, 0, 0, 0)
 
     def as_dict(self):
         return dict(model="gaussian", pos0=self.pos0, vel=self.vel, dT_peak=self.dT_peak,

@@ -8,7 +8,7 @@ import torch
 from pfkit import _lib
 from pfkit.allen_cahn import StateRHS
 from pfkit.config import make_params
-from problems import args, gaussian
+from problems import args, gaussian, quench, rosenthal
 
 FIELDS = ("m_g", "gamma", "kappa_g", "ad_hoc", "L0", "Qg", "gas_const", "T_liquidus", "T_clip", "zeta_sharpness",
           "anisotropy", "liquid_shift")
@@ -52,10 +52,11 @@ def test_values_without_the_defaults():
         make_params(dict(Nx=8, Ny=6, Nz=4), (1.0, 1.0, 1.0))
 
 
-def test_every_field_as_its_own_assignment():
+@pytest.mark.parametrize("make", [gaussian, rosenthal, lambda nx, ny, nz: quench(nz)], ids=["gaussian", "rosenthal", "quench"])
+def test_every_field_as_its_own_assignment(make):
     """The packed struct against one assignment per field, for every type that a yaml file or a program gives."""
     a = args(7, 5, 3, 9, force_liquid=True, T_liquidus="1623.5", m_g=np.float32(1.1), L0=3500, gamma=torch.tensor(0.75))
-    L = gaussian(7, 5, 3)
+    L = make(7, 5, 3)
     p = make_params(a, np.array([0.5, 1.5, 2.5]), L)
     q = _lib.ParamsT()
     q.nz, q.ny, q.nx, q.num_oris, q.force_liquid = 3, 5, 7, 9, 1
@@ -63,7 +64,14 @@ def test_every_field_as_its_own_assignment():
         q.h[d] = v
     for name in FIELDS:
         setattr(q, name, float(a[name]))
-    L.fill(q.laser)
+    q.laser.model = {"gaussian": _lib.PF_T_GAUSSIAN, "rosenthal": _lib.PF_T_ROSENTHAL, "quench": _lib.PF_T_QUENCH}[
+        L.as_dict()["model"]]
+    for name, v in L.as_dict().items():
+        if name in ("pos0", "dir"):
+            for d in range(3):
+                getattr(q.laser, name)[d] = v[d]
+        elif name != "model":
+            setattr(q.laser, name, v)
     assert bytes(p) == bytes(q)
     q = _lib.ParamsT()
     q.laser.model, q.laser.T_dtype = _lib.PF_T_BUFFER, _lib.PF_F64
