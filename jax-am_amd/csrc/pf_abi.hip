@@ -124,6 +124,8 @@ int make_stepdev(const pf_params_t* p, int dtype, const void* T_dev, const void*
 namespace {
 struct Tables {
   std::vector<StepEntry> t[3];
+  static constexpr int kMaxK = 32, kMaxTile = 8;
+  const StepEntry* at[3][kMaxK + 1][2][kMaxTile] = {};  // [dtype][K][anisotropic][tile]
   std::unique_ptr<std::atomic<int>[]> held[3];  // per entry and kernel (step, batch): workgroups the GPU holds at once (0: not asked yet)
   Tables() {
     using PartFn = const StepEntry* (*)(int*);
@@ -136,6 +138,8 @@ struct Tables {
       const StepEntry* e = f(&n);
       for (int i = 0; i < n; ++i) t[e[i].dtype].push_back(e[i]);
     }
+    for (int d = 0; d < 3; ++d)
+      for (const StepEntry& e : t[d]) at[d][e.k][e.aniso != 0][e.tile] = &e;
     for (int d = 0; d < 3; ++d) held[d] = std::make_unique<std::atomic<int>[]>(2 * t[d].size());
   }
 };
@@ -155,12 +159,9 @@ int entry_count(int dtype, int k, bool aniso) {
 }
 
 const StepEntry* find_entry(int dtype, int k, bool aniso, int tile) {
-  if (!valid_dtype(dtype)) return nullptr;
-  const Tables& tb = tables();
   if (tile < 0) tile = 0;
-  for (const StepEntry& e : tb.t[dtype])
-    if (e.k == k && (e.aniso != 0) == aniso && e.tile == tile) return &e;
-  return nullptr;
+  if (!valid_dtype(dtype) || k < 0 || k > Tables::kMaxK || tile >= Tables::kMaxTile) return nullptr;
+  return tables().at[dtype][k][aniso ? 1 : 0][tile];
 }
 
 // Asked of the runtime once per kernel.
@@ -234,17 +235,46 @@ static int deal_rows(const StepDev& a, int held) {
   return (most + cap - 1) / cap == (even + cap - 1) / cap;
 }
 
-static const StepEntry* choose_step(int dtype, int k, bool aniso, long long cells) {
-  if (small_step(dtype, k, cells)) return nullptr;
-  const bool odd = k % 2 != 0;
-  int tile;
-  if (dtype == PF_F64) tile = !odd ? 2 : k >= 17 ? 0 : 1;       // 16x4 lane pairs; 32x4; 16x4
-  else if (k % 4 == 0 && (k >= 16 || (dtype == PF_BF16 && k == 12 && cells < 2000000)))
-    tile = 4;  // 8x8 lane pairs (whole vectors in each half need K % 4 = 0; BF16 K = 12: 256x256x64 65.1 against 58.9 us)
-  else
-    tile = 2;  // 16x8
-  const StepEntry* e = find_entry(dtype, k, aniso, tile);
-  return e ? e : find_entry(dtype, k, aniso, 0);
+// Share of the GPU's workgroups that a launch of kernel e keeps busy: its marches, the shortest that fill the GPU a
+// whole number of times (fill_zchunk) but of two planes or more, against the fillings they take.
+static double filled(const StepEntry* e, int nz, int ny, int nx) {
+  const long long held = held_workgroups(e, false);
+  const long long cols = (long long)((nx + e->tx - 1) / e->tx) * ((ny + e->ty - 1) / e->ty);
+  const long long m = ((nz + 11) / 12 * cols + held - 1) / held;
+  const long long most = (nz + 1) / 2, k = m * held / cols < most ? m * held / cols : most;
+  return (double)(k * cols) / (double)(m * held);
+}
+
+// Flat grids in FP32 and BF16 (us, other tile / this one).  A single plane has nothing to march through and takes
+// the tile with the least halo, 32x8: 1024x1024x1, FP32 K = 16 52.7/48.0, BF16 K = 13 47.4/46.1, and the march of
+// channel groups only up to half as many values (64x2048x1, FP32 K = 13 10.5/8.3); so do up to four planes in BF16
+// for odd K where it fills the GPU as well: 512x512x3, K = 13 27.3/24.0.  Lane pairs lose to 16x8 tiles on few planes
+// if they keep under 0.7 of the GPU busy and those more: 256x256x8, two thirds, BF16 K = 16 20.3/16.4, 256x256x4, FP32
+// K = 20 15.4/14.3, 64x2048x2 16.5/13.8; but 300x700x6, 0.73, BF16 K = 20 33.8/38.9, and on more planes the marches are
+// cut to fill it (256x256x16, BF16 K = 16 28.5/29.0).
+static const StepEntry* choose_step(int dtype, int k, bool aniso, int nz, int ny, int nx) {
+  const long long cells = (long long)nz * ny * nx;
+  const bool odd = k % 2 != 0, bf16 = dtype == PF_BF16, flat = dtype != PF_F64 && nz == 1;
+  if (small_step(dtype, k, flat ? 2 * cells : cells)) return nullptr;
+  const StepEntry* wide = find_entry(dtype, k, aniso, 0);
+  const StepEntry* e = find_entry(dtype, k, aniso, 2);
+  if (dtype == PF_F64) {
+    e = find_entry(dtype, k, aniso, !odd ? 2 : k >= 17 ? 0 : 1);  // 16x4 lane pairs; 32x4; 16x4
+  } else if (flat) {
+    e = wide;
+  } else if (k % 4 == 0 && (k >= 16 || (bf16 && k == 12 && cells < 2000000))) {
+    // 8x8 lane pairs (whole vectors in each half need K % 4 = 0; BF16 K = 12: 256x256x64 65.1 against 58.9 us)
+    const StepEntry* pairs = find_entry(dtype, k, aniso, 4);
+    if (pairs && e && nz <= (bf16 ? 12 : 6)) {
+      const double share = filled(pairs, nz, ny, nx);
+      if (share >= 0.7 || share >= filled(e, nz, ny, nx)) e = pairs;
+    } else {
+      e = pairs;
+    }
+  } else if (bf16 && odd && nz <= 4 && e && wide && filled(wide, nz, ny, nx) >= filled(e, nz, ny, nx)) {
+    e = wide;
+  }
+  return e ? e : wide;  // 16x8
 }
 
 int default_zchunk(int nz, int ny, int nx, int tx, int ty) {
@@ -498,7 +528,7 @@ static int plan_step(const pf_params_t* p, int dtype, const void* T_dev, const v
     if (zchunk < 0 || (zchunk & ~(PF_ZCHUNK_TAIL | 0xffff)) != 0)
       return fail(PF_E_ARG, "zchunk must be a plane count in [0, 65535], optionally | PF_ZCHUNK_TAIL");
     if (march_fits(p, dtype)) return PF_E_ARG;
-    if (tile == -1) e = choose_step(dtype, p->num_oris, aniso, n);
+    if (tile == -1) e = choose_step(dtype, p->num_oris, aniso, p->nz, p->ny, p->nx);
   } else if (tile > 0 && entry_count(dtype, p->num_oris, aniso) > 0) {
     return fail(PF_E_ARG, "no such tile shape");
   }

@@ -34,6 +34,20 @@ def test_orders_of_tiles_are_bitwise_the_same(cuda, dtype, k, dims):
         assert torch.equal(o, outs[0])
 
 
+# each side of the library's choice of tile on few planes
+@pytest.mark.parametrize("dtype,k,dims", [
+    ("float32", 16, (300, 310, 1)), ("float32", 13, (201, 220, 1)), ("float32", 13, (64, 700, 1)), ("bfloat16", 13, (400, 403, 3)),
+    ("bfloat16", 13, (201, 203, 3)), ("bfloat16", 16, (250, 255, 8)), ("bfloat16", 16, (250, 255, 13)), ("float32", 20, (251, 249, 4)),
+    ("float32", 20, (251, 249, 7)), ("float32", 16, (300, 500, 6)), ("bfloat16", 12, (250, 251, 12)), ("float64", 16, (300, 310, 1))])
+def test_choice_on_few_planes_is_bitwise_the_same(cuda, dtype, k, dims):
+    s, eta = _states(cuda, *dims, k, dtype)
+    L = gaussian(*dims)
+    out, want = torch.full_like(eta, float("nan")), torch.full_like(eta, float("nan"))
+    s.state_rhs.step(eta, want, L, 0.1, 0.101, -2, 0)
+    s.state_rhs.step(eta, out, L, 0.1, 0.101, -1, 0)
+    assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("tile", [0, 1, 2])
 def test_one_long_row_of_tiles(cuda, tile):
     """A row of 19 million tiles: dealt by whole rows it would be padded to eight of them, past the largest launch."""
