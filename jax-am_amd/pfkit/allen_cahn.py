@@ -16,6 +16,7 @@ import time
 
 import numpy as np
 import torch
+import torch.autograd.forward_ad as forward_ad
 
 from . import _lib
 from .config import make_params, with_defaults
@@ -129,14 +130,20 @@ def explicit_euler(state_pre, t_crt, f, ode_params):
     return (y, t_crt), y
 
 
+def _tracked(*values):
+    """Whether autograd, in reverse or in forward mode, follows one of these."""
+    return any(isinstance(v, torch.Tensor) and (v.requires_grad and torch.is_grad_enabled() or
+                                                forward_ad.unpack_dual(v).tangent is not None) for v in values)
+
+
 def rk4(state_pre, t_crt, f, ode_params):
     """allen_cahn.py:90-103 (classical RK4): four stage kernels that form the combinations of the
     right-hand sides as they compute them (pf_rk4), or four pf_rhs evaluations where f is not a
-    plain StateRHS, has more orientations than those kernels take, or the state is tracked by autograd
-    (which then follows the combination of the stages)."""
+    plain StateRHS, has more orientations than those kernels take, or the state or a time is tracked by
+    autograd (which then follows the combination of the stages)."""
     y_prev, t_prev = state_pre
     y_prev = f.check_state(y_prev)
-    if type(f) is StateRHS and not y_prev.requires_grad:
+    if type(f) is StateRHS and not _tracked(y_prev, t_prev, t_crt):
         T, = ode_params
         y = f.rk4_step(y_prev, T, t_prev, t_crt)
         if y is not None:
