@@ -82,7 +82,8 @@ class BatchEngine:
     def add(self, inst: Instance) -> int:
         a = with_defaults(inst.pf_args)
         tdt = inst.torch_dtype
-        self.stream.wait_stream(torch.cuda.current_stream(self.device))  # inputs made on the caller's stream
+        caller = torch.cuda.current_stream(self.device)
+        self.stream.wait_stream(caller)  # inputs made on the caller's stream
         cdt = torch.float64 if tdt == torch.float64 else torch.float32
         with torch.cuda.stream(self.stream):
             b0 = torch.empty((inst.N, inst.K), dtype=tdt, device=self.device)
@@ -99,6 +100,9 @@ class BatchEngine:
                                                    inst.K, self.stream.cuda_stream), "pf_init_onehot")
             axes = torch.as_tensor(np.ascontiguousarray(inst.grain_dirs), dtype=cdt, device=self.device) \
                 if float(a["anisotropy"]) > 0 else None
+        # the engine's stream reads the caller's tensors, maybe behind steps queued there, and writes the first state:
+        # what the caller queues next (a write to those tensors, a read of that state) comes after
+        caller.wait_stream(self.stream)
         bi = _lib.BatchInstT()
         bi.eta_dev[0] = b0.data_ptr()
         bi.eta_dev[1] = b1.data_ptr()
@@ -143,7 +147,7 @@ class BatchEngine:
             bi.path_dev = None
         bi.p = make_params(a, inst.h_xyz, laser)
         inst.params = bi.p
-        self.stream.wait_stream(torch.cuda.current_stream(self.device))  # the table is copied on the caller's stream
+        self.stream.wait_stream(caller)  # the table is copied on the caller's stream
         slot = self.lib.pf_batch_add(self.h, ctypes.byref(bi))
         if slot < 0:
             _lib.check(slot, "pf_batch_add")

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from pfkit import PFSolver, workloads
+from pfkit.allen_cahn import DTYPES
 from pfkit.batch import BatchEngine
 from pfkit.laser import RosenthalRamp
 
@@ -120,4 +121,45 @@ def test_source_tables_are_planned_per_step(cuda, chunk):
         else:
             want = _solo(w, n)
         assert left[s] == 0 and torch.equal(eng.state(s, par[s]), want)
+    eng.close()
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("side", [False, True])
+def test_admission_while_steps_are_queued_takes_the_state_of_its_call(cuda, dtype, side):
+    """One buffer refilled in place for each of several requests, admitted behind a long queue of steps: every instance
+    starts from what the buffer held at its own add.  The first state is there for the caller's next reads."""
+    busy = _make(0, 128, 128, 64, 20, "float32", 300)
+    W = [_make(1 + j, 40, 31, 17, 6, dtype, 3) for j in range(4)]
+    eng = BatchEngine(max_instances=16)
+    eng.add(busy.instance())
+    eng.run(16, 16)
+    caller = torch.cuda.Stream() if side else torch.cuda.current_stream()
+    states = [torch.rand(w.N, w.K, device=cuda, generator=torch.Generator(cuda).manual_seed(j)).to(DTYPES[dtype])
+              for j, w in enumerate(W)]
+    oris = [torch.as_tensor(w.polycrystal.cell_ori_inds, device=cuda, dtype=torch.int32) for w in W]
+    eta0, ori = torch.empty_like(states[0]), torch.empty_like(oris[0])
+    caller.wait_stream(torch.cuda.current_stream())
+    got, first = [], []
+    with torch.cuda.stream(caller):
+        for w, state, o in zip(W, states, oris):
+            eng.run(32, 16)
+            eta0.copy_(state)
+            ori.copy_(o)
+            for kw in (dict(eta0=eta0), dict()):
+                inst = w.instance(**kw)
+                if not kw:
+                    inst.cell_ori_inds = ori
+                got.append(eng.add(inst))
+                first.append(eng.state(got[-1], 0).clone())
+            eta0.fill_(float("nan"))
+            ori.fill_(0)
+    torch.cuda.current_stream().wait_stream(caller)
+    eng.run_to_completion()
+    par = eng.status()[2]
+    for j, w in enumerate(W):
+        s = PFSolver(w.pf_args, w.polycrystal, dtype=w.dtype, clean=False, tile=-2, zchunk=0)
+        for slot, start, e in zip(got[2 * j:], first[2 * j:], (states[j], s.ini_cond())):
+            assert torch.equal(start, e)
+            assert torch.equal(eng.state(slot, par[slot]), s.run(e, w.ts(3), w.laser))
     eng.close()
