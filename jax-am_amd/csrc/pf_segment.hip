@@ -161,8 +161,7 @@ constexpr int MZ = 16;     // planes of a moments tile (SX x SY columns)
 constexpr int MSLOT = 64;  // grains of a tile summed in LDS; those past them go straight to memory
 
 __global__ __launch_bounds__(ST) void seg_zero_kernel(unsigned long long* __restrict__ p, long long n) {
-  const long long i = (long long)blockIdx.x * ST + threadIdx.x;
-  if (i < n) p[i] = 0;
+  for (long long i = (long long)blockIdx.x * ST + threadIdx.x; i < n; i += (long long)gridDim.x * ST) p[i] = 0;
 }
 
 __device__ __forceinline__ void seg_flush(unsigned long long* mom, int32_t g, const long long (&s)[NMOM],
@@ -237,6 +236,7 @@ static SegTiles seg_tiles(const pf_params_t* p) {
   g.mtiles = (long long)g.tx * g.ty * ((p->nz + MZ - 1) / MZ);
   return g;
 }
+// blocks of a loop over tiles (a launch has fewer than 2^32 threads)
 static unsigned seg_blocks(long long tiles) { return (unsigned)(tiles < (1 << 20) ? tiles : 1 << 20); }
 
 }  // namespace pf
@@ -279,7 +279,7 @@ int pf_segment_moments(const int32_t* labels_dev, const int32_t* cid_dev, const 
   hipStream_t s = (hipStream_t)stream;
   const SegTiles g = seg_tiles(p);
   const long long nm = (long long)n_grains * NMOM;
-  seg_zero_kernel<<<(unsigned)((nm + ST - 1) / ST), ST, 0, s>>>((unsigned long long*)moments_dev, nm);
+  seg_zero_kernel<<<seg_blocks((nm + ST - 1) / ST), ST, 0, s>>>((unsigned long long*)moments_dev, nm);
   seg_moments_kernel<<<seg_blocks(g.mtiles), ST, 0, s>>>(g, labels_dev, cid_dev, (unsigned long long*)moments_dev);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? PF_OK : hip_fail(e, "pf_segment_moments");

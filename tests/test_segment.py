@@ -150,3 +150,31 @@ def test_labels_across_tiles(cuda, nx, ny, nz, k, kind):
         cols = [np.ones_like(x), x, y, z, x * x, y * y, z * z, x * y, x * z, y * z]
         ref = np.stack([np.bincount(cid[labels[c]], v, ng.value) for v in cols], axis=1).astype(np.int64)
         assert np.array_equal(mom.cpu().numpy(), ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ng", [1, 30_000_001, 2 ** 32 // 10 + 5])
+def test_moments_of_very_many_grains(cuda, ng):
+    """More moments than a launch has threads (2^32; 34 GB), and than its blocks clear in one turn: zero but for the
+    rows of the grains that have cells."""
+    import torch
+    from pfkit import _lib
+    from pfkit.config import make_params
+    nx, ny, nz = 5, 3, 2
+    p = make_params(args(nx, ny, nz, 2), (1.0, 1.0, 1.0), None)
+    labels = torch.zeros(nx * ny * nz, dtype=torch.int32, device=cuda)
+    labels[nx * ny:] = 20
+    cid = torch.zeros(nx * ny * nz, dtype=torch.int32, device=cuda)
+    cid[20] = ng - 1
+    mom = torch.full((ng, 10), -5, dtype=torch.int64, device=cuda)
+    _lib.check(_lib.load().pf_segment_moments(labels.data_ptr(), cid.data_ptr(), p, ng, mom.data_ptr(),
+                                              _lib.stream_handle(cuda)), "moments")
+    z, y, x = np.unravel_index(np.arange(nx * ny * nz), (nz, ny, nx))
+    cols = np.stack([np.ones_like(x), x, y, z, x * x, y * y, z * z, x * y, x * z, y * z], axis=1)
+    halves = cols[:nx * ny].sum(0), cols[nx * ny:].sum(0)
+    if ng == 1:
+        assert np.array_equal(mom[0].cpu().numpy(), halves[0] + halves[1])
+    else:
+        assert np.array_equal(mom[0].cpu().numpy(), halves[0]) and np.array_equal(mom[-1].cpu().numpy(), halves[1])
+        for part in mom[1:-1].split(1 << 26):
+            assert not bool(part.any())
