@@ -131,7 +131,8 @@ int pf_step(const void* eta_in_dev, void* eta_out_dev, int32_t dtype, const void
  * array of steps + 1 times, read before the call returns) with the same temperature argument; the states
  * go eta_in_dev -> buf0_dev -> buf1_dev -> buf0_dev ..., so the result is in buf0_dev for odd
  * `steps` and in buf1_dev for even ones, and eta_in_dev is only read.  The three buffers must not
- * alias.  Other arguments as pf_step.
+ * alias, except that eta_in_dev may be buf1_dev (a run that goes on from an earlier one's result;
+ * it is then overwritten from step 2 on).  Other arguments as pf_step.
  */
 int pf_run(const void* eta_in_dev, void* buf0_dev, void* buf1_dev, int32_t dtype, const void* T_dev,
            const pf_params_t* p, const void* axes_dev, const double* ts, int32_t steps, int32_t tile, int32_t zchunk,

@@ -610,8 +610,9 @@ int pf_run(const void* eta_in_dev, void* buf0_dev, void* buf1_dev, int32_t dtype
            const pf_params_t* p, const void* axes_dev, const double* ts, int32_t steps, int32_t tile, int32_t zchunk,
            void* stream) {
   if (!eta_in_dev || !buf0_dev || !buf1_dev || !ts) return fail(PF_E_ARG, "NULL argument");
-  if (eta_in_dev == buf0_dev || eta_in_dev == buf1_dev || buf0_dev == buf1_dev)
-    return fail(PF_E_ARG, "eta_in and the two buffers must not alias");
+  // eta_in may be buf1: step 1 has read it before step 2 writes it
+  if (eta_in_dev == buf0_dev || buf0_dev == buf1_dev)
+    return fail(PF_E_ARG, "buf0 must alias neither eta_in nor buf1");
   if (((uintptr_t)eta_in_dev | (uintptr_t)buf0_dev | (uintptr_t)buf1_dev) & 15)
     return fail(PF_E_ARG, "eta buffers must be 16-byte aligned");
   if (steps < 1) return fail(PF_E_ARG, "steps must be >= 1");

@@ -26,6 +26,9 @@ DTYPES = {"float64": torch.float64, "float32": torch.float32, "bfloat16": torch.
           "f64": torch.float64, "f32": torch.float32, "bf16": torch.bfloat16}
 
 
+RUN_BLOCK = 256  # steps that PFSolver.run launches in one native call (an interrupt takes effect between calls)
+
+
 def _as_dtype(d):
     if d is None:
         return torch.float64
@@ -229,10 +232,14 @@ class PFSolver:
             ts = [float(t) for t in ts]
         times = np.ascontiguousarray(ts, dtype=np.float64)
         p, Tptr = rhs.params_for(T)
-        _lib.check(_lib.load().pf_run(eta.data_ptr(), bufs[0].data_ptr(), bufs[1].data_ptr(), rhs.pf_dtype, Tptr, p,
-                                      _lib.ptr(rhs.axes), times.ctypes.data, n, int(self.tile), int(self.zchunk),
-                                      _lib.stream_handle(self.device)), "pf_run")
-        return bufs[(n - 1) % 2]
+        for i in range(0, n, RUN_BLOCK):
+            m = min(RUN_BLOCK, n - i)
+            _lib.check(_lib.load().pf_run(eta.data_ptr(), bufs[0].data_ptr(), bufs[1].data_ptr(), rhs.pf_dtype, Tptr, p,
+                                          _lib.ptr(rhs.axes), times[i:].ctypes.data, m, int(self.tile), int(self.zchunk),
+                                          _lib.stream_handle(self.device)), "pf_run")
+            eta = bufs[(m - 1) % 2]
+            bufs = bufs[m % 2], eta
+        return eta
 
     def run_toolpath(self, eta0, toolpath, steps=None, callback=None):
         """Advance along a source table: a ``pfkit.laser.Toolpath`` (multi_scan/example.py:88-105) or

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from pfkit import PFSolver
+from pfkit.allen_cahn import RUN_BLOCK
 from problems import args, gaussian, poly
 
 pytestmark = pytest.mark.gpu
@@ -42,3 +43,15 @@ def test_parameters_changed_between_calls_take_effect(cuda):
     got = s.run(eta, [0.1, 0.101], L)
     want = PFSolver(dict(a, m_g=2.5), pc, dtype="float64", device=cuda, clean=False).run(eta, [0.1, 0.101], L)
     assert torch.equal(got, want) and not torch.equal(got, first)
+
+
+@pytest.mark.parametrize("dtype,extra", [("float32", 1), ("bfloat16", 2)])
+def test_a_run_of_several_blocks(cuda, dtype, extra):
+    nx, ny, nz, k = 13, 9, 6, 5
+    s = PFSolver(args(nx, ny, nz, k, anisotropy=0.15), poly(nx, ny, nz, k), dtype=dtype, device=cuda, clean=False)
+    n = 2 * RUN_BLOCK + extra
+    ts, L, eta0 = 0.1 + np.arange(n + 1) * 1e-4, gaussian(nx, ny, nz), s.ini_cond()
+    want = eta0
+    for i in range(n):
+        (want, _), _ = s.stepper((want, ts[i]), ts[i + 1], [L])
+    assert torch.equal(s.run(eta0, ts, L), want) and torch.equal(eta0, s.ini_cond())
