@@ -72,6 +72,7 @@ class StateRHS:
         p.laser.model = _lib.PF_T_BUFFER
         p.laser.T_dtype = _lib.TORCH_TO_PF[Tt.dtype]
         self._T_keep = Tt  # alive until the stream has consumed it (stream order + caching allocator)
+        p.T_buffer = Tt    # and while p is in use: another thread's call on this object may replace _T_keep
         return p, Tt.data_ptr()
 
     def check_state(self, eta):

@@ -1,7 +1,9 @@
 """CPU tests of how PFSolver.run hands a long run to pf_run: blocks that go on from each other, and a Ctrl-C that takes
 effect between them.  A stand-in for the native call applies pf_run's contract to host memory."""
 import ctypes
+import gc
 import signal
+import weakref
 from types import SimpleNamespace
 
 import numpy as np
@@ -56,6 +58,28 @@ def test_an_interrupt_takes_effect_between_blocks(solver):
     with pytest.raises(KeyboardInterrupt):
         solver.run(torch.zeros(24, 3, dtype=torch.float64), np.arange(50 * RUN_BLOCK + 1.0), gaussian(4, 3, 2))
     assert len(solver.calls) == 2
+
+
+def test_a_run_holds_its_temperature(solver):
+    """The converted copy of a temperature array stays while the run's blocks read it, also if another call on the same
+    solver (another thread's) converts one of its own between them."""
+    held = []
+
+    class Between:
+        def __init__(self, pf_run):
+            self.pf_run = pf_run
+
+        def __call__(self, *a):
+            held.append(held[0] if held else weakref.ref(solver.state_rhs._T_keep))
+            solver.state_rhs.params_for(np.zeros(24, np.float16))
+            gc.collect()
+            assert held[-1]() is not None
+            return self.pf_run(*a)
+
+    lib = SimpleNamespace(pf_run=Between(allen_cahn._lib.load().pf_run))
+    allen_cahn._lib.load = lambda: lib
+    solver.run(torch.zeros(24, 3, dtype=torch.float64), np.arange(2 * RUN_BLOCK + 1.0), np.full(24, 900.0, np.float16))
+    assert len(held) == 2 and held[0]() is None
 
 
 def test_pf_run_refuses_aliased_buffers_without_gpu():
