@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from pfkit import PFSolver, workloads
+from pfkit._lib import PFError
 from pfkit.allen_cahn import DTYPES
 from pfkit.batch import BatchEngine
 from pfkit.laser import RosenthalRamp
@@ -81,19 +82,34 @@ def test_classes_and_parts_that_run_side_by_side(cuda, ks, dtype, chunk):
     eng.close()
 
 
+def _quad_items(dims, k, v=4):
+    """Work items of instances of one class on the march of channel groups, as rebuild_work counts them."""
+    up = lambda a, b: -(-a // b)  # noqa: E731
+    c = 256 // up(k, v)
+    runs = [up(up(nx * ny, c), 8) * 8 for nx, ny, _ in dims]
+    chunks = max(1, 1024 // sum(runs))
+    return sum(r * up(nz, min(up(nz, chunks), 512 // c)) for r, (_, _, nz) in zip(runs, dims))
+
+
 def test_more_work_items_than_max_tiles(cuda):
-    """Slots are charged as they asked to be tiled; shorter marches and channel groups make more work items than that,
-    and the work list grows (between replays of graphs that held the shorter one)."""
-    W = [_make(j, 33, 31, 24, 25, "float32", 20) for j in range(3)]
-    charge = (33 * 31 * 24 + 255) // 256
-    eng = BatchEngine(max_instances=4, max_tiles=3 * charge)
+    """Slots are charged as they asked to be tiled; shorter marches and channel groups make more work items than that.
+    The list of a tiny instance fits and a graph that holds it has run; with two more of the class (the same graph
+    key) it grows past max_tiles, and the next replay must not read the old one."""
+    dims, k = [(6, 6, 4), (33, 31, 24), (33, 31, 24)], 25
+    W = [_make(j, *d, k, "float32", 20) for j, d in enumerate(dims)]
+    charge = sum(-(-nx * ny * nz // 256) for nx, ny, nz in dims)
+    assert _quad_items(dims[:1], k) <= charge < _quad_items(dims, k)
+    eng = BatchEngine(max_instances=4, max_tiles=charge)
     slots = [eng.add(W[0].instance())]
     eng.run(4, 4)
     slots += [eng.add(w.instance()) for w in W[1:]]
-    eng.run(4, 4)
-    par = eng.status()[2]
-    for w, s, n in zip(W, slots, (8, 4, 4)):
-        assert torch.equal(eng.state(s, par[s]), _solo(w, n))
+    for n in (4, 8):
+        eng.run(4, 4)
+        par = eng.status()[2]
+        for w, s, done in zip(W, slots, (4 + n, n, n)):
+            assert torch.equal(eng.state(s, par[s]), _solo(w, done))
+    with pytest.raises(PFError, match="max_tiles"):
+        eng.add(_make(9, 33, 31, 24, k, "float32", 20).instance())
     eng.close()
 
 

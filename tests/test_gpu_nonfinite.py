@@ -13,7 +13,7 @@ import pytest
 import torch
 
 from oracle import pf_oracle as O
-from pfkit import PFSolver, workloads
+from pfkit import PFSolver, _lib, workloads
 from pfkit.batch import BatchEngine
 from pfkit.serve import Request, Server
 from problems import args, gaussian, poly
@@ -44,7 +44,9 @@ def test_nan_in_eta_spreads_like_the_oracle(dtype, eps, cuda):
     with np.errstate(invalid="ignore"):
         ref = O.explicit_euler(eta, t0, t1, T, a, pc.mesh_h_xyz, pc.unique_grain_directions)
     s = PFSolver(a, pc, dtype=dtype, device=cuda, clean=False)
-    for tile, zc in ((s.tile, s.zchunk), (-2, 0)):   # the fused tiled kernel and the generic kernel
+    pf = _lib.TORCH_TO_PF[dtype]
+    # the library's choice, the march of channel groups and every tiled kernel
+    for tile, zc in [(s.tile, s.zchunk), (-2, 0)] + [(t, 5) for t in range(_lib.load().pf_tile_count(pf, K))]:
         x = torch.as_tensor(eta, dtype=dtype, device=cuda)
         out = torch.empty_like(x)
         s.state_rhs.step(x, out, L, t0, t1, tile, zc)
@@ -67,11 +69,12 @@ def test_nan_temperature_spreads_like_the_oracle(cuda):
     with np.errstate(invalid="ignore"):
         ref = O.explicit_euler(eta, t0, t1, T, a, pc.mesh_h_xyz, pc.unique_grain_directions)
     for dtype in (torch.float64, torch.float32):
-        s = PFSolver(a, pc, dtype=dtype, device=cuda, clean=False)
-        (out, _), _ = s.stepper((torch.as_tensor(eta, dtype=dtype, device=cuda), t0), t1, [T])
-        got = out.double().cpu().numpy()
-        assert np.array_equal(np.isnan(got), np.isnan(ref)), dtype
-        assert np.array_equal(np.flatnonzero(np.isnan(ref).any(axis=1)), [77])
+        for tile in [-1, -2] + list(range(_lib.load().pf_tile_count(_lib.TORCH_TO_PF[dtype], K))):
+            s = PFSolver(a, pc, dtype=dtype, device=cuda, clean=False, tile=tile, zchunk=0)
+            (out, _), _ = s.stepper((torch.as_tensor(eta, dtype=dtype, device=cuda), t0), t1, [T])
+            got = out.double().cpu().numpy()
+            assert np.array_equal(np.isnan(got), np.isnan(ref)), (dtype, tile)
+            assert np.array_equal(np.flatnonzero(np.isnan(ref).any(axis=1)), [77])
 
 
 def test_server_fails_the_nan_request_alone(cuda):
