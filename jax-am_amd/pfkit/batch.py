@@ -147,7 +147,8 @@ class BatchEngine:
             bi.path_dev = None
         bi.p = make_params(a, inst.h_xyz, laser)
         inst.params = bi.p
-        self.stream.wait_stream(caller)  # the table is copied on the caller's stream
+        if path is not None:
+            self.stream.wait_stream(caller)  # the table is copied on the caller's stream
         slot = self.lib.pf_batch_add(self.h, ctypes.byref(bi))
         if slot < 0:
             _lib.check(slot, "pf_batch_add")
