@@ -227,9 +227,9 @@ bool small_step(int dtype, int k, long long cells) {
 // K = 20, FP32 85.0/91.4, 300x100x80 85.3/91.6, 100x300x40 48.3/51.3); a filling more costs far more than
 // that (320x72x48, 36 rows of 40 tiles, 192 held per XCD: 54.9/44.8; 200x56x64, K = 17, 77 rows of 13, 128 held:
 // 35.8/33.9), and so do XCDs without work (4096x32x1, K = 20, 4 rows: 16.5/10.4).
-static int deal_rows(const StepDev& a, int held) {
+static bool deal_rows(const StepDev& a, int held) {
   const long long rows = (long long)a.tiles_y * a.tiles_z;
-  if (rows < 8) return 0;
+  if (rows < 8) return false;
   const long long most = (rows + 7) / 8 * a.tiles_x, even = (rows * a.tiles_x + 7) / 8;
   const long long cap = held >= 8 ? held / 8 : 1;
   return (most + cap - 1) / cap == (even + cap - 1) / cap;
@@ -536,7 +536,7 @@ static int plan_step(const pf_params_t* p, int dtype, const void* T_dev, const v
     const long long cols = (long long)((p->nx + e->tx - 1) / e->tx) * ((p->ny + e->ty - 1) / e->ty);
     if ((zchunk & 0xffff) == 0) zchunk |= fill_zchunk(p->nz, cols, held_workgroups(e, false));
     set_tiles(a, e->tx, e->ty, zchunk);
-    a.rows = deal_rows(a, held_workgroups(e, false));
+    a.rsh = deal_rows(a, held_workgroups(e, false)) ? 3 : 0;
     if (tile_launch(a) >= (1LL << 31)) return fail(PF_E_ARG, "too many tiles");
     fn = e->step;
   } else {

@@ -102,7 +102,7 @@ struct StepDev {
   int tiles_x, tiles_y, tiles_z, zc;
   int zs, zsplit;      // planes [0, zsplit) in chunks of zs, [zsplit, nz) in chunks of zc (zsplit 0: no tail)
   int tmodel, t_f64, force_liquid;
-  int rows;            // 1: a step's tiles go to the XCDs by whole rows (tile_coords)
+  int rsh;             // a step's tiles go to the XCDs by whole rows (3) or one by one (0): tile_coords
   float ihx2f, ihy2f, ihz2f, Bf;          // FP32 copies of ihx2, ihy2, ihz2, B
   double hx, hy, hz;
   double ihx2, ihy2, ihz2;
@@ -1262,7 +1262,8 @@ template <class TS, int V, bool TAIL> struct QuadAt {
 // threads, into an LDS table.  One barrier per plane.  Same per-cell and per-channel arithmetic as
 // the tiled march: results are bitwise the same.
 // 97x101x45, K = 33, FP32, anisotropic: 1336 us with one thread per cell (7 value-by-value strided
-// reads per channel), 46 us here (3.1e11 updates/s; reading and writing the state once takes 19 us);
+// reads per channel), 43.7 us here (3.3e11 updates/s; the kernel takes 40 us with the state in the last-level cache, 46
+// without; reading and writing the state once takes 19 us);
 // pf_rhs on 96x80x40, K = 16, FP64: 415 us against 24 us.  Bound by its VALU work, about 90
 // instructions per channel: a wavefront's lanes hold different channels, so that a channel that is
 // zero everywhere can not be skipped as the tiled march does it (256x256x64, K = 20, FP32: 197 us
@@ -1513,36 +1514,31 @@ __device__ __forceinline__ void generic_cell(const StepDev& a, const StepDyn& dy
   }
 }
 
-// Tile order of a launch: layers of z-chunks from the top of the domain down.  Workgroups are
-// dispatched in index order and dealt round-robin to the 8 XCDs, so the top layer, where a
+// Tile order of a launch: rows of tiles, layer by layer of z-chunks from the top of the domain down.
+// Workgroups are dispatched in index order and dealt round-robin to the 8 XCDs, so the top layer, where a
 // surface heat source makes cells hot and the per-cell FP64 path slow, starts first and the
-// cheaper layers below fill in behind it.  Two ways to deal a layer:
-//   a.rows: workgroup t takes the next tile of row 8m + (t mod 8), the rows of all layers counted
-//     together: every XCD walks whole rows of tiles, so the x-neighbours of a tile (whose halo columns it
-//     re-reads) run on the same XCD and share its L2.  The rows are padded to a multiple of 8 (false for a
-//     workgroup past the last one); an XCD's share is whole rows, up to one row more than an even share;
-//   else as item_coords deals an instance's tiles, no padding, shares that differ by one tile.
+// cheaper layers below fill in behind it.  The rows of all layers are counted together, and
+//   rsh = 3: workgroup t takes the next tile of row 8m + (t mod 8): every XCD walks whole rows of tiles, so the
+//     x-neighbours of a tile (whose halo columns it re-reads) run on the same XCD and share its L2.  The rows are
+//     padded to a multiple of 8 (false for a workgroup past the last one); an XCD's share is whole rows, up to one
+//     row more than an even share;
+//   rsh = 0: workgroup t takes tile t, x fastest: no padding, shares that differ by one tile.
 // deal_rows (pf_abi.hip) chooses.
 __host__ __device__ inline long long tile_launch(const StepDev& a) {
-  const long long rows = (long long)a.tiles_y * a.tiles_z;
-  return (a.rows ? (rows + 7) / 8 * 8 : rows) * a.tiles_x;
+  const long long rows = (long long)a.tiles_y * a.tiles_z, turn = 1LL << a.rsh;
+  return (rows + turn - 1) / turn * turn * a.tiles_x;
 }
-__device__ __forceinline__ void item_coords(int t, int tiles_x, int tiles_y, int tiles_z, int& tx, int& ty, int& tz);
 __device__ __forceinline__ bool tile_coords(const StepDev& a, int t, int& tx, int& ty, int& tz) {
-  if (!a.rows) {
-    item_coords(t, a.tiles_x, a.tiles_y, a.tiles_z, tx, ty, tz);
-    return true;
-  }
-  const int i = t >> 3, m = i / a.tiles_x;
+  const int i = t >> a.rsh, m = i / a.tiles_x;
   tx = i - m * a.tiles_x;
-  const int row = 8 * m + (t & 7), layer = row / a.tiles_y;
+  const int row = (m << a.rsh) + (t & ((1 << a.rsh) - 1)), layer = row / a.tiles_y;
   ty = row - layer * a.tiles_y;
   tz = a.tiles_z - 1 - layer;
   return tz >= 0;
 }
 
-// Tile t of a grid whose layers follow each other without padding (a work item of the batch engine, a launch
-// that is not dealt by rows): whole rows to an XCD in layers whose rows divide by 8, else x fastest, then y (64 instances of 32^3 to 128x128x64: 4.27e11 updates/s,
+// The same for a work item of the batch engine: an instance's layers follow each other without padding, and
+// only layers whose rows divide by 8 are dealt by rows (64 instances of 32^3 to 128x128x64: 4.27e11 updates/s,
 // with every instance dealt by padded rows 4.14e11).
 __device__ __forceinline__ void item_coords(int t, int tiles_x, int tiles_y, int tiles_z, int& tx, int& ty, int& tz) {
   const int nl = tiles_x * tiles_y;
