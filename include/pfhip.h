@@ -242,10 +242,11 @@ int pf_reduce_noalloc(const void* eta_dev, int32_t dtype, const void* T_dev, con
  * Batched engine: many independent instances (uneven grids, K, dtype) advanced
  * together by persistent launches over a device-resident tile work list, captured
  * into a HIP graph of `chunk` steps.  No counterpart in the reference (which runs
- * one solve per process); each instance follows the same per-step arithmetic as
- * pf_step with the same tile shape, so its result is bitwise the same alone and in
- * the mix.  The engine allocates its tables once at creation; eta buffers are the
- * caller's.  See pf_batch_* below.
+ * one solve per process); every kernel the engine may choose for an instance gives
+ * bitwise the step of pf_step, so its result is the same alone and in the mix.
+ * The engine allocates its tables once at creation, except the work list: it grows
+ * (16 bytes an item) where the marches chosen for the current instances make more
+ * items than max_tiles.  Eta buffers are the caller's.  See pf_batch_* below.
  */
 typedef struct pf_batch pf_batch_t;
 
@@ -271,9 +272,12 @@ typedef struct pf_batch_inst {
   const double* path_dev;
 } pf_batch_inst_t;
 
+/* max_instances slots; max_tiles bounds the instances in them by the work items that they ask for (tiles of their own
+ * tile and zchunk, or blocks of 256 cells for K without tiled kernels): pf_batch_add refuses past it. */
 pf_batch_t* pf_batch_create(int32_t max_instances, int32_t max_tiles, void* stream);
 void pf_batch_destroy(pf_batch_t* b);
-/* Put an instance into a free slot; returns the slot index (>= 0) or a PF_E* code. */
+/* Put an instance into a free slot; returns the slot index (>= 0) or a PF_E* code.  Does not wait: what the instance
+ * points to is read by the engine's stream from here on. */
 int pf_batch_add(pf_batch_t* b, const pf_batch_inst_t* inst);
 /* Free a slot (its steps may be unfinished; the caller owns the buffers). */
 int pf_batch_remove(pf_batch_t* b, int32_t slot);

@@ -14,9 +14,9 @@
 //     into one HIP graph and replayed.  Graphs are cached by (chunk, set of classes with
 //     work and their kernels): admitting or removing an instance only rewrites table entries and work
 //     lists, and a new capture happens only for a class set not seen before.
-// Every tile of an instance runs exactly the per-cell arithmetic of pf_step with the
-// same tile shape, so an instance's trajectory does not depend on what else is in
-// the batch.
+// The kernel and march length of an instance may change from rebuild to rebuild as others of its class come
+// and go.  Its trajectory does not: every kernel (tile shape, lane split, channel groups, one thread per cell) and
+// every march length gives bitwise the same step (test_gpu_parity, test_gpu_anyk, test_gpu_batch_blocks).
 #include <string.h>
 
 #include <algorithm>

@@ -6,9 +6,11 @@
 // the per-cell quantities (sum of squares, argmax) are combined through LDS by one thread per cell.
 //   argmax, 256x256x64, K = 20, FP32: 62 us, 5.7 TB/s, the rate of a copy (one thread per cell reading
 //   its row value by value: 256 us; BF16 34 us, FP64 on half the cells 61 us).
-//   reduce, the same state: 134 us (a thread per cell with its three neighbour rows, a second
-//   pass for the volumes and one block adding up the partials: 1648 + 1593 + 1463 us).  Its FP64
-//   arithmetic, about 14 instructions per value, takes half of that, the reads 57 us.
+//   reduce, the same state: 127 us (a thread per cell with its three neighbour rows, a second
+//   pass for the volumes and one block adding up the partials: 1648 + 1593 + 1463 us).  Bound by the
+//   issue of VALU instructions, 46 a value, which keep the SIMDs busy 83 % of the time: 14 are FP64
+//   arithmetic, 4 conversions, 8 integer arithmetic, the rest the compares and selects of argmax and
+//   finiteness and copies.  The reads take 57 us, LDS bank conflicts 5 % of the time.
 #include <math.h>
 
 #include <mutex>
@@ -449,8 +451,9 @@ int pf_argmax(const void* eta_dev, int32_t dtype, int64_t n_cells, int32_t k, in
   return err == hipSuccess ? PF_OK : hip_fail(err, "pf_argmax launch");
 }
 
-// The partial results of the blocks; at least the size of the tables of ceil(n / 2048) rows and
-// ceil(n / 4096) column sums that callers have sized their workspaces by.
+// The partial results of the blocks, at most 1024 of them: 0.4 MB for K = 20, 3.2 MB for K = 256.  Never
+// less than the tables of ceil(n / 2048) rows and ceil(n / 4096) column sums of an earlier layout, so that the grids
+// that pf_reduce_noalloc refuses for their size stay the same.
 size_t pf_reduce_workspace_bytes(int64_t n_cells, int32_t k) {
   if (n_cells < 1 || k < 1) return 0;
   long long rows = (n_cells + 2047) / 2048;
