@@ -12,7 +12,16 @@ from typing import Tuple
 
 from . import _lib
 
-_LASER = struct.Struct("@2i18d")  # pf_laser_t; one call sets all fields (a step is launched every few microseconds)
+_LASER = struct.Struct("@2i18d")  # pf_laser_t
+
+
+def _fill(L, *values):
+    """All fields of the pf_laser_t L by one call (a step is launched every few microseconds)."""
+    try:
+        _LASER.pack_into(L, 0, *values)
+    except struct.error as e:
+        raise TypeError(f"a source parameter is not a number: {e}") from None
+
 
 @dataclass
 class Rosenthal:
@@ -40,8 +49,8 @@ class Rosenthal:
 
     def fill(self, L):
         p, d = self.pos0, self.dir
-        _LASER.pack_into(L, 0, _lib.PF_T_ROSENTHAL, 0, self.T_ambient, p[0], p[1], p[2], d[0], d[1], d[2], self.vel,
-                         self.Q, self.kappa_T, self.alpha, self.T_cap, 0, 0, 0, 0, 0, 0)
+        _fill(L, _lib.PF_T_ROSENTHAL, 0, self.T_ambient, p[0], p[1], p[2], d[0], d[1], d[2], self.vel,
+              self.Q, self.kappa_T, self.alpha, self.T_cap, 0, 0, 0, 0, 0, 0)
 
     def as_dict(self):
         return dict(model="rosenthal", pos0=self.pos0, vel=self.vel, Q=self.Q, alpha=self.alpha,
@@ -62,8 +71,8 @@ class Gaussian:
 
     def fill(self, L):
         p, d = self.pos0, self.dir
-        _LASER.pack_into(L, 0, _lib.PF_T_GAUSSIAN, 0, self.T_ambient, p[0], p[1], p[2], d[0], d[1], d[2], self.vel,
-                         0, 0, 0, 0, self.dT_peak, self.sigma_xy, self.sigma_z, 0, 0, 0)
+        _fill(L, _lib.PF_T_GAUSSIAN, 0, self.T_ambient, p[0], p[1], p[2], d[0], d[1], d[2], self.vel,
+              0, 0, 0, 0, self.dT_peak, self.sigma_xy, self.sigma_z, 0, 0, 0)
 
     def as_dict(self):
         return dict(model="gaussian", pos0=self.pos0, vel=self.vel, dT_peak=self.dT_peak,

@@ -76,3 +76,12 @@ def test_every_field_as_its_own_assignment(make):
     q = _lib.ParamsT()
     q.laser.model, q.laser.T_dtype = _lib.PF_T_BUFFER, _lib.PF_F64
     assert bytes(make_params(a, (1.0, 1.0, 1.0)))[-_lib.ParamsT.laser.size:] == bytes(q.laser)
+
+
+@pytest.mark.parametrize("make,name", [(gaussian, "sigma_z"), (rosenthal, "Q"), (rosenthal, "vel"), (lambda nx, ny, nz: quench(nz), "T_ref")])
+@pytest.mark.parametrize("value", [None, "300", 1j])
+def test_a_source_parameter_that_is_no_number_is_a_type_error(make, name, value):
+    L = make(7, 5, 3)
+    setattr(L, name, value)
+    with pytest.raises(TypeError):
+        make_params(args(7, 5, 3, 9), (1.0, 1.0, 1.0), L)
